@@ -16,200 +16,266 @@ namespace kore {
 // ---------------------------------------------------------------------------
 // batched complex GEMM
 // ---------------------------------------------------------------------------
-// Workgroup = 4 waves, output tile 64x64, each wave a 32x32 quadrant made of
-// 2x2 MFMA 16x16 tiles; K staged through LDS in slabs of GT_K = 16 (32 measured
+// Workgroup = 4 waves, output tile 32 S x 32 S, each wave a quadrant of S x S
+// MFMA 16x16 tiles; K staged through LDS in slabs of GT_K = 16 (32 measured
 // slower: the larger LDS and register footprint halves the workgroups per CU).
-constexpr int GT_M = 64, GT_N = 64, GT_K = 16;
-constexpr int GT_EPT = GT_K * GT_M / 256;   // slab elements of A (and of B) per thread
-constexpr int GT_PADB = 1;
+// S = 1 or 2 by gemm_small_tiles below.
+constexpr int GT_K = 16;
+// complex64 double-buffers its slabs in LDS (one barrier per slab); two slabs
+// of complex128 would leave room for two workgroups per CU where three fit
+template <class T> constexpr int GT_NBUF = sizeof(T) == 4 ? 2 : 1;
+template <class T, int S> struct GemmLds {
+  cx<T> A[GT_NBUF<T>][GT_K][32 * S];
+  cx<T> B[GT_NBUF<T>][32 * S][GT_K + 1];
+};
 
-// One 64 x 64 tile of C = alpha sum_p A_p B_p + beta C for the workgroup
-// (256 threads); sA / sB are the workgroup's LDS staging.
-template <class T>
-__device__ __forceinline__ void gemm_tile_body(const GemmDesc<T>& d, const int tile, cx<T> (&sA)[GT_K][GT_M],
-                                               cx<T> (&sB)[GT_N][GT_K + GT_PADB]) {
+// Global load of base[off] with a uniform base: one 32-bit offset register
+// and no address arithmetic per load.
+template <class T> __device__ __forceinline__ cx<T> gld_at(const cx<T>* base, unsigned off) {
+  typedef typename cx_vec<T>::type V;
+  const V v = *(const __attribute__((address_space(1))) V*)((const __attribute__((address_space(1))) char*)base +
+                                                            (size_t)off * sizeof(cx<T>));
+  return cx<T>{v.x, v.y};
+}
+
+// One tile of C = alpha sum_p A_p B_p + beta C for the workgroup (256
+// threads).  A and B tiles wholly or partly outside the matrices read their
+// last row or column instead (rows and columns of C that are not stored), so
+// that only the last slab of a product has anything to check: its missing k
+// count as zero.
+template <class T, int S>
+__device__ __forceinline__ void gemm_tile_body(const GemmDesc<T>& d, const int tile, GemmLds<T, S>& sm) {
   using A4 = typename acc4<T>::type;
+  constexpr int TS = 32 * S, NQ = 2 * S;      // tile edge, slab elements of A (and of B) per thread
+  constexpr int NBUF = GT_NBUF<T>;
   const int tid = threadIdx.x;
   const int lane = tid & 63;
-  const int wave = tid >> 6;
-  const int wr = (wave >> 1) * 32, wc = (wave & 1) * 32;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wr = (wave >> 1) * 16 * S, wc = (wave & 1) * 16 * S;
   const int l16 = lane & 15, lq = lane >> 4;
-  {
-    const int i0 = (tile % d.tiles_m) * GT_M;
-    const int j0 = (tile / d.tiles_m) * GT_N;
-    // 16 x 16 sub-tiles wholly outside C (edge tiles of sizes that are not
-    // multiples of 64, e.g. 200 = 3*64 + 8) are skipped, wave-uniformly
-    const bool rv0 = i0 + wr < d.m, rv1 = i0 + wr + 16 < d.m;
-    const bool cv0 = j0 + wc < d.n, cv1 = j0 + wc + 16 < d.n;
-    // complex64: three real products per complex step (Karatsuba's 3M
-    // form): cre = sum ar br, cim = sum ai bi, csum = sum (ar + ai)(br + bi),
-    // and at the end re = cre - cim, im = csum - cre - cim: 3/4 of the
-    // matrix-core work of the four-product form, with a normwise error bound
-    // of the same order (Higham, Accuracy and Stability of Numerical
-    // Algorithms, section 23.2.4); the complex64 factor is a preconditioner
-    // whose answers FP64 refinement or GMRES corrects.  complex128 keeps the
-    // four products (cre, cim = real and imaginary parts): measured, the 3M
-    // form makes the FP64 factor 10 % faster at N = 500 but moves the most
-    // ill-conditioned MAC eigenvalues (relative condition 1e16) further from
-    // the oracle's than the four-product form does.
-    constexpr bool k3m = sizeof(T) == 4;
-    A4 cre[2][2], cim[2][2], csum[2][2];
+  const int tiles_m = (d.m + TS - 1) / TS;
+  const int i0 = (tile % tiles_m) * TS;
+  const int j0 = (tile / tiles_m) * TS;
+  // 16 x 16 sub-tiles wholly outside C (edge tiles of sizes that are not
+  // multiples of the tile, e.g. 200 = 3*64 + 8) are skipped, wave-uniformly
+  bool rv[S], cv[S];
 #pragma unroll
-    for (int a = 0; a < 2; ++a)
+  for (int s = 0; s < S; ++s) {
+    rv[s] = i0 + wr + 16 * s < d.m;
+    cv[s] = j0 + wc + 16 * s < d.n;
+  }
+  // complex64: three real products per complex step (Karatsuba's 3M
+  // form): cre = sum ar br, cim = sum ai bi, csum = sum (ar + ai)(br + bi),
+  // and at the end re = cre - cim, im = csum - cre - cim: 3/4 of the
+  // matrix-core work of the four-product form, with a normwise error bound
+  // of the same order (Higham, Accuracy and Stability of Numerical
+  // Algorithms, section 23.2.4); the complex64 factor is a preconditioner
+  // whose answers FP64 refinement or GMRES corrects.  complex128 keeps the
+  // four products (cre, cim = real and imaginary parts): measured, the 3M
+  // form makes the FP64 factor 10 % faster at N = 500 but moves the most
+  // ill-conditioned MAC eigenvalues (relative condition 1e16) further from
+  // the oracle's than the four-product form does.
+  constexpr bool k3m = sizeof(T) == 4;
+  A4 cre[S][S], cim[S][S], csum[S][S];
 #pragma unroll
-      for (int b = 0; b < 2; ++b) {
-        cre[a][b] = A4{0, 0, 0, 0};
-        cim[a][b] = A4{0, 0, 0, 0};
-        csum[a][b] = A4{0, 0, 0, 0};
-      }
+  for (int a = 0; a < S; ++a)
+#pragma unroll
+    for (int b = 0; b < S; ++b) {
+      cre[a][b] = A4{0, 0, 0, 0};
+      cim[a][b] = A4{0, 0, 0, 0};
+      csum[a][b] = A4{0, 0, 0, 0};
+    }
 
-    // Slabs of GT_K k-columns over the (up to two) products, register
-    // double-buffered: slab s+1 is requested from memory before slab s is
-    // multiplied, so the load latency hides behind the matrix-core work.
-    cx<T> ra[GT_EPT], rb[GT_EPT];
-    auto load = [&](int p, int k0) {      // selects, not indexing: d stays in registers
-      const cx<T>* __restrict__ A = p ? d.A[1] : d.A[0];
-      const cx<T>* __restrict__ B = p ? d.B[1] : d.B[0];
-      const int K = p ? d.k[1] : d.k[0];
-      const int64_t lda = p ? d.lda[1] : d.lda[0], ldb = p ? d.ldb[1] : d.ldb[0];
-      if (d.opA == 0) {        // A slab element (k = tid / (64/EPT), i = EPT (tid % (64/EPT)) + q)
-        const int gk = k0 + tid / (GT_M / GT_EPT), ii = (tid % (GT_M / GT_EPT)) * GT_EPT;
+  // Slabs of GT_K k-columns over the (up to two) products, register
+  // double-buffered: slab s+1 is requested from memory before slab s is
+  // multiplied, so the load latency hides behind the matrix-core work.
+  // Thread (kt = tid / 16, l16) loads A[i0 + l16 + 16 q][k0 + kt] and
+  // B[k0 + l16][j0 + kt + 16 q]: 16 lanes read consecutive addresses of
+  // both, and write consecutive LDS words.
+  const int kt = tid >> 4;
+  cx<T> ra[NQ], rb[NQ];
+  unsigned oa[NQ], ob[NQ];                    // element offsets of the thread from the product's base
+  const cx<T>* __restrict__ A = nullptr;      // base of the next slab (uniform)
+  const cx<T>* __restrict__ B = nullptr;
+  int K = 0;
+  int64_t lda = 0;
+  auto start = [&](int p) {                   // product p (selects, not indexing: d stays in registers)
+    K = p ? d.k[1] : d.k[0];
+    lda = p ? d.lda[1] : d.lda[0];
+    const int64_t ldb = p ? d.ldb[1] : d.ldb[0];
+    A = (p ? d.A[1] : d.A[0]) + i0;
+    B = (p ? d.B[1] : d.B[0]) + (int64_t)j0 * ldb;
 #pragma unroll
-        for (int q = 0; q < GT_EPT; ++q) {
-          const int gi = i0 + ii + q;
-          ra[q] = czero<T>();
-          if (gk < K && gi < d.m) ra[q] = gld(A + (int64_t)gk * lda + gi);
-        }
-      } else {                 // A_eff(i,k) = conj(A_store(k,i)), A_store column-major K x m
-        const int gi = i0 + (tid >> 2), kk = (tid & 3) * GT_EPT;
+    for (int q = 0; q < NQ; ++q) {
+      oa[q] = (unsigned)min(l16 + 16 * q, d.m - 1 - i0) + (unsigned)kt * (unsigned)lda;
+      ob[q] = (unsigned)min(kt + 16 * q, d.n - 1 - j0) * (unsigned)ldb + (unsigned)l16;
+    }
+  };
+  auto load = [&](int k0) {                   // the slab at k0; A, B move to the next one
+    const int rem = K - k0;
+    if (rem >= GT_K) {
 #pragma unroll
-        for (int q = 0; q < GT_EPT; ++q) {
-          const int gk = k0 + kk + q;
-          ra[q] = czero<T>();
-          if (gk < K && gi < d.m) {
-            ra[q] = gld(A + (int64_t)gi * lda + gk);
-            ra[q].im = -ra[q].im;
-          }
-        }
+      for (int q = 0; q < NQ; ++q) ra[q] = gld_at<T>(A, oa[q]);
+#pragma unroll
+      for (int q = 0; q < NQ; ++q) rb[q] = gld_at<T>(B, ob[q]);
+    } else {                                  // the product's last slab, rem of 16 columns
+      const bool ka = kt < rem, kb = l16 < rem;
+#pragma unroll
+      for (int q = 0; q < NQ; ++q) {
+        ra[q] = gld_at<T>(A, ka ? oa[q] : oa[q] - (unsigned)(kt - rem + 1) * (unsigned)lda);
+        rb[q] = gld_at<T>(B, kb ? ob[q] : ob[q] - (unsigned)(l16 - rem + 1));
+        if (!ka) ra[q] = czero<T>();
+        if (!kb) rb[q] = czero<T>();
       }
-      const int gj = j0 + (tid >> 2), kk = (tid & 3) * GT_EPT;   // B slab element (j, k)
+    }
+    A += (int64_t)GT_K * lda;
+    B += GT_K;
+  };
+  auto valid = [&](int p) { return d.A[p] != nullptr && d.k[p] > 0; };
+  int p = valid(0) ? 0 : (valid(1) ? 1 : 2), k0 = 0, buf = 0;
+  if (p < 2) {
+    start(p);
+    load(0);
+  }
+  while (p < 2) {
+    const int rem = K - k0;
+    if (NBUF == 1) __syncthreads();           // the previous slab has been consumed
 #pragma unroll
-      for (int q = 0; q < GT_EPT; ++q) {
-        const int gk = k0 + kk + q;
-        rb[q] = czero<T>();
-        if (gk < K && gj < d.n) rb[q] = gld(B + (int64_t)gj * ldb + gk);
+    for (int q = 0; q < NQ; ++q) {
+      sm.A[buf][kt][l16 + 16 * q] = ra[q];
+      sm.B[buf][kt + 16 * q][l16] = rb[q];
+    }
+    __syncthreads();
+    int pn = p;
+    k0 += GT_K;                               // next slab
+    if (k0 >= K) {
+      pn = (p == 0 && valid(1)) ? 1 : 2;
+      k0 = 0;
+      if (pn < 2) start(pn);
+    }
+    if (pn < 2) load(k0);
+#pragma unroll
+    for (int kk = 0; kk < GT_K; kk += 4) {
+      if (kk >= rem) break;                   // uniform
+      cx<T> a[S], b[S];
+#pragma unroll
+      for (int s = 0; s < S; ++s) {
+        a[s] = sm.A[buf][kk + lq][wr + 16 * s + l16];
+        b[s] = sm.B[buf][wc + 16 * s + l16][kk + lq];
       }
-    };
-    auto valid = [&](int p) { return d.A[p] != nullptr && d.k[p] > 0; };
-    int p = valid(0) ? 0 : (valid(1) ? 1 : 2), k0 = 0;
-    if (p < 2) load(p, 0);
-    while (p < 2) {
-      __syncthreads();                      // the previous slab has been consumed
-      if (d.opA == 0) {
-        const int kk = tid / (GT_M / GT_EPT), ii = (tid % (GT_M / GT_EPT)) * GT_EPT;
+      if constexpr (k3m) {
+        T as[S], bs[S];
 #pragma unroll
-        for (int q = 0; q < GT_EPT; ++q) sA[kk][ii + q] = ra[q];
+        for (int q = 0; q < S; ++q) {
+          as[q] = a[q].re + a[q].im;
+          bs[q] = b[q].re + b[q].im;
+        }
+#pragma unroll
+        for (int rs = 0; rs < S; ++rs)
+#pragma unroll
+          for (int cs = 0; cs < S; ++cs)
+            if (rv[rs] && cv[cs]) {
+              cre[rs][cs] = mfma16(b[cs].re, a[rs].re, cre[rs][cs]);
+              cim[rs][cs] = mfma16(b[cs].im, a[rs].im, cim[rs][cs]);
+              csum[rs][cs] = mfma16(bs[cs], as[rs], csum[rs][cs]);
+            }
       } else {
-        const int ii = tid >> 2, kk = (tid & 3) * GT_EPT;
 #pragma unroll
-        for (int q = 0; q < GT_EPT; ++q) sA[kk + q][ii] = ra[q];
+        for (int rs = 0; rs < S; ++rs)
+#pragma unroll
+          for (int cs = 0; cs < S; ++cs)
+            if (rv[rs] && cv[cs]) cmma<T>(cre[rs][cs], cim[rs][cs], a[rs], b[cs]);
       }
-      {
-        const int jj = tid >> 2, kk = (tid & 3) * GT_EPT;
-#pragma unroll
-        for (int q = 0; q < GT_EPT; ++q) sB[jj][kk + q] = rb[q];
-      }
-      __syncthreads();
-      int pn = p, kn = k0 + GT_K;           // next slab
-      if (kn >= (p ? d.k[1] : d.k[0])) {
-        pn = (p == 0 && valid(1)) ? 1 : 2;
-        kn = 0;
-      }
-      if (pn < 2) load(pn, kn);
-#pragma unroll
-      for (int kk = 0; kk < GT_K; kk += 4) {
-        cx<T> a[2], b[2];
-#pragma unroll
-        for (int s = 0; s < 2; ++s) {
-          a[s] = sA[kk + lq][wr + 16 * s + l16];
-          b[s] = sB[wc + 16 * s + l16][kk + lq];
-        }
-        if constexpr (k3m) {
-          T as[2], bs[2];
-#pragma unroll
-          for (int q = 0; q < 2; ++q) {
-            as[q] = a[q].re + a[q].im;
-            bs[q] = b[q].re + b[q].im;
-          }
-#pragma unroll
-          for (int rs = 0; rs < 2; ++rs)
-#pragma unroll
-            for (int cs = 0; cs < 2; ++cs)
-              if ((rs ? rv1 : rv0) && (cs ? cv1 : cv0)) {
-                cre[rs][cs] = mfma16(b[cs].re, a[rs].re, cre[rs][cs]);
-                cim[rs][cs] = mfma16(b[cs].im, a[rs].im, cim[rs][cs]);
-                csum[rs][cs] = mfma16(bs[cs], as[rs], csum[rs][cs]);
-              }
-        } else {
-#pragma unroll
-          for (int rs = 0; rs < 2; ++rs)
-#pragma unroll
-            for (int cs = 0; cs < 2; ++cs)
-              if ((rs ? rv1 : rv0) && (cs ? cv1 : cv0)) cmma<T>(cre[rs][cs], cim[rs][cs], a[rs], b[cs]);
-        }
-      }
-      p = pn;
-      k0 = kn;
     }
-    __syncthreads();                        // LDS is reused by the next tile
-    // epilogue: lane holds C[i0+wr+16rs+l16][j0+wc+16cs+mfma_mrow(lq,r)].
-    // Per row sub-tile, the eight old values of C are loaded together before
-    // any store, so that their latencies overlap (a load after a store to a
-    // possibly aliasing address would wait for the previous one).
-    const bool acc = d.beta != T(0);
+    p = pn;
+    if (NBUF == 2) buf ^= 1;
+  }
+  __syncthreads();                            // LDS is reused by the next tile
+  // epilogue: lane holds C[i0+wr+16rs+l16][j0+wc+16cs+mfma_mrow(lq,r)].
+  // Per row sub-tile, the old values of C are loaded together before
+  // any store, so that their latencies overlap (a load after a store to a
+  // possibly aliasing address would wait for the previous one).
+  const bool acc = d.beta != T(0);
 #pragma unroll
-    for (int rs = 0; rs < 2; ++rs) {
-      const int gi = i0 + wr + 16 * rs + l16;
-      cx<T> o[2][4];
+  for (int rs = 0; rs < S; ++rs) {
+    const int gi = i0 + wr + 16 * rs + l16;
+    cx<T> o[S][4];
 #pragma unroll
-      for (int cs = 0; cs < 2; ++cs)
+    for (int cs = 0; cs < S; ++cs)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int gj = j0 + wc + 16 * cs + mfma_mrow<T>(lq, r);
-          o[cs][r] = czero<T>();
-          if (acc && gi < d.m && gj < d.n) o[cs][r] = gld(d.C + (int64_t)gj * d.ldc + gi);
-        }
+      for (int r = 0; r < 4; ++r) {
+        const int gj = j0 + wc + 16 * cs + mfma_mrow<T>(lq, r);
+        o[cs][r] = czero<T>();
+        if (acc && gi < d.m && gj < d.n) o[cs][r] = gld(d.C + (int64_t)gj * d.ldc + gi);
+      }
 #pragma unroll
-      for (int cs = 0; cs < 2; ++cs)
+    for (int cs = 0; cs < S; ++cs)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int gj = j0 + wc + 16 * cs + mfma_mrow<T>(lq, r);
-          if (gi < d.m && gj < d.n) {
-            T vre = cre[rs][cs][r], vim = cim[rs][cs][r];
-            if constexpr (k3m) {
-              vre = cre[rs][cs][r] - cim[rs][cs][r];
-              vim = csum[rs][cs][r] - cre[rs][cs][r] - cim[rs][cs][r];
-            }
-            cx<T> v{d.alpha * vre, d.alpha * vim};
-            if (acc) {
-              v.re += d.beta * o[cs][r].re;
-              v.im += d.beta * o[cs][r].im;
-            }
-            gst(d.C + (int64_t)gj * d.ldc + gi, v);
+      for (int r = 0; r < 4; ++r) {
+        const int gj = j0 + wc + 16 * cs + mfma_mrow<T>(lq, r);
+        if (gi < d.m && gj < d.n) {
+          T vre = cre[rs][cs][r], vim = cim[rs][cs][r];
+          if constexpr (k3m) {
+            vre = cre[rs][cs][r] - cim[rs][cs][r];
+            vim = csum[rs][cs][r] - cre[rs][cs][r] - cim[rs][cs][r];
           }
+          cx<T> v{d.alpha * vre, d.alpha * vim};
+          if (acc) {
+            v.re += d.beta * o[cs][r].re;
+            v.im += d.beta * o[cs][r].im;
+          }
+          gst(d.C + (int64_t)gj * d.ldc + gi, v);
         }
-    }
+      }
   }
 }
 
-template <class T>
-__global__ __launch_bounds__(256, 3) void gemm_batched_kernel(const GemmDesc<T>* __restrict__ descs) {
-  const GemmDesc<T> d = descs[blockIdx.y];
-  const int ntiles = d.tiles_m * d.tiles_n;
-  if ((int)blockIdx.x >= ntiles) return;
-  __shared__ cx<T> sA[GT_K][GT_M];
-  __shared__ cx<T> sB[GT_N][GT_K + GT_PADB];
-  for (int tile = blockIdx.x; tile < ntiles; tile += gridDim.x) gemm_tile_body<T>(d, tile, sA, sB);
+// Workgroup id -> (item, part of the item), for launches of `per` workgroups per
+// item.  Consecutive workgroups go to the chip's eight dies in turn, each with
+// its own L2: all parts of an item are kept on one die, so that what
+// they share is fetched into one L2 and not into eight.  That needs many items
+// (a few would leave dies idle): 64 and more.  Measured, complex128 products:
+// 298 of 200 rows 583 -> 520 us, 298 of 500 rows 5.22 -> 5.07 ms.
+constexpr int XCD_MIN_ITEMS = 64;
+__device__ __forceinline__ void xcd_item(int id, int per, int nitems, int& item, int& part) {
+  if (nitems >= XCD_MIN_ITEMS) {
+    const int slot = id >> 3;
+    item = (slot / per) * 8 + (id & 7);
+    part = slot % per;
+  } else {
+    item = id / per;
+    part = id % per;
+  }
+}
+static inline unsigned xcd_grid(int items, int per) {
+  return (unsigned)(items >= XCD_MIN_ITEMS ? (items + 7) / 8 * 8 : items) * (unsigned)per;
+}
+
+// Tile edge 32 instead of 64: where it covers much less padding (n = 200: 224
+// rows instead of 256; n = 150: 160 instead of 192), and where the launch holds
+// few tiles, so that four times the workgroups fill the chip.  Measured, us per
+// launch of one n x n x n product per item, edge 64 / 32:
+//   complex128  n = 500: 1 item 85 / 33, 8 items 155 / 155, 32 items 618 / 649
+//               n = 200: 1 item 36 / 14, 32 items 68 / 65, 150 items 257 / 226
+//               n = 374: 16 items 165 / 133, 32 items 273 / 255, 64 items 512 / 529
+//               n = 450 (480 rows instead of 512): 64 items 1019 / 1032
+//   complex64   n = 500: 1 item 49 / 22, 4 items 54 / 45, 8 items 74 / 83
+//               n = 150: 32 items 26 / 21, 150 items 68 / 55
+//               n = 450: 64 items 434 / 485
+template <class T> static bool gemm_small_tiles(int nitems, int t64, int t32) {
+  return t32 < 3.2 * t64 || (int64_t)nitems * t64 < (sizeof(T) == 8 ? 1536 : 384);
+}
+
+template <class T, int S>
+__global__ __launch_bounds__(256, 3) void gemm_batched_kernel(const GemmDesc<T>* __restrict__ descs, int ndesc,
+                                                              int per) {
+  __shared__ GemmLds<T, S> sm;
+  int di, tile;
+  xcd_item(blockIdx.x, per, ndesc, di, tile);
+  if (di >= ndesc) return;
+  const GemmDesc<T> d = descs[di];
+  const int ntiles = ((d.m + 32 * S - 1) / (32 * S)) * ((d.n + 32 * S - 1) / (32 * S));
+  for (; tile < ntiles; tile += per) gemm_tile_body<T, S>(d, tile, sm);
 }
 
 template <class T> __device__ __forceinline__ T tiny_pivot() { return sizeof(T) == 8 ? T(1e-150) : T(1e-18); }
@@ -716,19 +782,22 @@ __global__ __launch_bounds__(NT) void gj_panel_kernel(const InvDesc<T>* __restri
 // outer panel outside J (pivot rows cleared by the panel kernel), on the
 // batched GEMM's tile with descriptors made here (columns [q0, p0), then
 // [p0 + w, q0 + wo)); K = w <= 32.
-template <class T>
-__global__ __launch_bounds__(256, 3) void gj_update_kernel(const InvDesc<T>* __restrict__ descs, int p0) {
-  __shared__ cx<T> sA[GT_K][GT_M];
-  __shared__ cx<T> sB[GT_N][GT_K + GT_PADB];
-  const InvDesc<T> v = descs[blockIdx.y];
+template <class T, int S>
+__global__ __launch_bounds__(256, 3) void gj_update_kernel(const InvDesc<T>* __restrict__ descs, int ndesc, int per,
+                                                           int p0) {
+  constexpr int TS = 32 * S;
+  __shared__ GemmLds<T, S> sm;
+  int di, t;
+  xcd_item(blockIdx.x, per, ndesc, di, t);
+  if (di >= ndesc) return;
+  const InvDesc<T> v = descs[di];
   const int n = v.n;
   if (p0 >= n) return;
   int q0, wo;
   gj_outer_range(n, p0, q0, wo);
   const int w = min(GJM_WP, n - p0);
   const int n0 = p0 - q0, n1 = q0 + wo - (p0 + w);
-  const int tm = (n + 63) / 64, tn0 = (n0 + 63) / 64, tn1 = (n1 + 63) / 64;
-  int t = blockIdx.x;
+  const int tm = (n + TS - 1) / TS, tn0 = (n0 + TS - 1) / TS, tn1 = (n1 + TS - 1) / TS;
   if (t >= tm * (tn0 + tn1)) return;      // uniform over the workgroup
   int jstart = q0, ncols = n0;
   if (t >= tm * tn0) {
@@ -749,12 +818,9 @@ __global__ __launch_bounds__(256, 3) void gj_update_kernel(const InvDesc<T>* __r
   d.ldc = v.ld;
   d.m = n;
   d.n = ncols;
-  d.opA = 0;
-  d.tiles_m = tm;
-  d.tiles_n = (ncols + 63) / 64;
   d.alpha = T(1);
   d.beta = T(1);
-  gemm_tile_body<T>(d, t, sA, sB);
+  gemm_tile_body<T, S>(d, t, sm);
 }
 
 // phase 0: S[l n + k] = M[r_k, r^{-1}(l)];  phase 1: M <- S.   Grid: (column chunks, blocks).
@@ -823,16 +889,20 @@ __global__ __launch_bounds__(256) void gj_outer_gather_kernel(const InvDesc<T>* 
 
 // M[:, j] += M[:, O] R_O[:, j] for the columns outside O: the batched GEMM's
 // tile on descriptors made here (columns [0, q0), then [q0 + wo, n)).
-template <class T>
-__global__ __launch_bounds__(256, 3) void gj_outer_update_kernel(const InvDesc<T>* __restrict__ descs, int q0) {
-  __shared__ cx<T> sA[GT_K][GT_M];
-  __shared__ cx<T> sB[GT_N][GT_K + GT_PADB];
-  const InvDesc<T> v = descs[blockIdx.y];
+template <class T, int S>
+__global__ __launch_bounds__(256, 3) void gj_outer_update_kernel(const InvDesc<T>* __restrict__ descs, int ndesc,
+                                                                 int per, int q0) {
+  constexpr int TS = 32 * S;
+  __shared__ GemmLds<T, S> sm;
+  int di, t;
+  xcd_item(blockIdx.x, per, ndesc, di, t);
+  if (di >= ndesc) return;
+  const InvDesc<T> v = descs[di];
   const int n = v.n;
   if (n < GJ_OUTER_MIN || q0 >= n) return;
   const int wo = min(GJ_WO, n - q0);
-  const int tm = (n + 63) / 64, tn0 = (q0 + 63) / 64, n1 = n - q0 - wo, tn1 = (n1 + 63) / 64;
-  int t = blockIdx.x;
+  const int n1 = n - q0 - wo;
+  const int tm = (n + TS - 1) / TS, tn0 = (q0 + TS - 1) / TS, tn1 = (n1 + TS - 1) / TS;
   if (t >= tm * (tn0 + tn1)) return;      // uniform over the workgroup
   int jstart = 0, ncols = q0;
   if (t >= tm * tn0) {
@@ -853,12 +923,28 @@ __global__ __launch_bounds__(256, 3) void gj_outer_update_kernel(const InvDesc<T
   d.ldc = v.ld;
   d.m = n;
   d.n = ncols;
-  d.opA = 0;
-  d.tiles_m = tm;
-  d.tiles_n = (ncols + 63) / 64;
   d.alpha = T(1);
   d.beta = T(1);
-  gemm_tile_body<T>(d, t, sA, sB);
+  gemm_tile_body<T, S>(d, t, sm);
+}
+
+template <class T, int S>
+static void launch_gj_updates(const InvDesc<T>* d_descs, int ndesc, int nmax, int p0, hipStream_t s) {
+  constexpr int TS = 32 * S;
+  const int nt = (nmax + TS - 1) / TS;
+  // column tiles of the two ranges an update covers: at most 128 / TS + 1 in
+  // an outer panel of 128 columns, at most nt + 1 in a block below
+  // GJ_OUTER_MIN rows (whichever is more when a launch holds both)
+  const int ntb = ((nmax < GJ_OUTER_MIN ? nmax : GJ_OUTER_MIN) + TS - 1) / TS + 1;
+  const int per = nt * (nmax >= GJ_OUTER_MIN && ntb < GJ_WO / TS + 1 ? GJ_WO / TS + 1 : ntb);
+  hipLaunchKernelGGL((gj_update_kernel<T, S>), dim3(xcd_grid(ndesc, per)), dim3(256), 0, s, d_descs, ndesc, per, p0);
+}
+
+template <class T, int S>
+static void launch_gj_outer_updates(const InvDesc<T>* d_descs, int ndesc, int nmax, int q0, hipStream_t s) {
+  const int nt = (nmax + 32 * S - 1) / (32 * S), per = nt * nt;
+  hipLaunchKernelGGL((gj_outer_update_kernel<T, S>), dim3(xcd_grid(ndesc, per)), dim3(256), 0, s, d_descs, ndesc, per,
+                     q0);
 }
 
 template <class T>
@@ -870,18 +956,18 @@ static hipError_t launch_gj_inverse_multi(const InvDesc<T>* d_descs, int ndesc, 
                          d_descs, p0);
     else
       hipLaunchKernelGGL((gj_panel_kernel<T, 512, 512>), dim3(ndesc), dim3(512), 0, s, d_descs, p0);
-    // column tiles of the two ranges an update covers: at most 3 in an outer
-    // panel of 128 columns, at most nt + 1 in a block below GJ_OUTER_MIN rows
-    // (at most 5 when such a block shares a launch with larger ones)
-    const int ntc = nmax >= GJ_OUTER_MIN ? 5 : nt + 1;
-    hipLaunchKernelGGL((gj_update_kernel<T>), dim3(nt * ntc, ndesc), dim3(256), 0, s, d_descs, p0);
+    // the columns an update covers come in multiples of 32 (a panel's width)
+    launch_gj_updates<T, 1>(d_descs, ndesc, nmax, p0, s);
     // the end of an outer panel (of every block whose outer panel holds p0)
     const int pe = p0 + GJM_WP;
     if (nmax >= GJ_OUTER_MIN && (pe % GJ_WO == 0 || pe >= nmax)) {
       const int q0 = (p0 / GJ_WO) * GJ_WO;
       const int chunks = (nmax * GJ_WO + 255) / 256 < 256 ? (nmax * GJ_WO + 255) / 256 : 256;
       hipLaunchKernelGGL((gj_outer_gather_kernel<T>), dim3(chunks, ndesc), dim3(256), 0, s, d_descs, q0);
-      hipLaunchKernelGGL((gj_outer_update_kernel<T>), dim3(nt * nt, ndesc), dim3(256), 0, s, d_descs, q0);
+      if (gemm_small_tiles<T>(ndesc, nt * nt, 4 * nt * nt))
+        launch_gj_outer_updates<T, 1>(d_descs, ndesc, nmax, q0, s);
+      else
+        launch_gj_outer_updates<T, 2>(d_descs, ndesc, nmax, q0, s);
     }
   }
   const int nc = (nmax + 15) / 16;
@@ -894,10 +980,14 @@ static hipError_t launch_gj_inverse_multi(const InvDesc<T>* d_descs, int ndesc, 
 // launchers
 // ---------------------------------------------------------------------------
 template <class T>
-hipError_t launch_gemm_batched(const GemmDesc<T>* d_descs, int ndesc, int max_tiles, hipStream_t s) {
-  if (ndesc <= 0 || max_tiles <= 0) return hipSuccess;
-  dim3 grid(max_tiles, ndesc);
-  hipLaunchKernelGGL(gemm_batched_kernel<T>, grid, dim3(256), 0, s, d_descs);
+hipError_t launch_gemm_batched(const GemmDesc<T>* d_descs, int ndesc, GemmTiles t, hipStream_t s) {
+  if (ndesc <= 0 || t.t64 <= 0) return hipSuccess;
+  if (gemm_small_tiles<T>(ndesc, t.t64, t.t32))
+    hipLaunchKernelGGL((gemm_batched_kernel<T, 1>), dim3(xcd_grid(ndesc, t.t32)), dim3(256), 0, s, d_descs, ndesc,
+                       t.t32);
+  else
+    hipLaunchKernelGGL((gemm_batched_kernel<T, 2>), dim3(xcd_grid(ndesc, t.t64)), dim3(256), 0, s, d_descs, ndesc,
+                       t.t64);
   return hipGetLastError();
 }
 
@@ -926,8 +1016,8 @@ hipError_t launch_gj_inverse(const InvDesc<T>* d_descs, int ndesc, int nmin, int
   return hipGetLastError();
 }
 
-template hipError_t launch_gemm_batched<double>(const GemmDesc<double>*, int, int, hipStream_t);
-template hipError_t launch_gemm_batched<float>(const GemmDesc<float>*, int, int, hipStream_t);
+template hipError_t launch_gemm_batched<double>(const GemmDesc<double>*, int, GemmTiles, hipStream_t);
+template hipError_t launch_gemm_batched<float>(const GemmDesc<float>*, int, GemmTiles, hipStream_t);
 template hipError_t launch_gj_inverse<double>(const InvDesc<double>*, int, int, int, hipStream_t);
 template hipError_t launch_gj_inverse<float>(const InvDesc<float>*, int, int, int, hipStream_t);
 

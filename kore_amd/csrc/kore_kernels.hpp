@@ -7,16 +7,13 @@ namespace kore {
 
 template <class T> struct cx;
 
-// C = beta*C + alpha*(op(A1)*B1 + op(A2)*B2); column-major; op = identity
-// (opA = 0) or conjugate transpose of a K x m stored A (opA = 1).
+// C = beta*C + alpha*(A1*B1 + A2*B2); column-major.
 template <class T> struct GemmDesc {
   const cx<T>* A[2];
   const cx<T>* B[2];
   cx<T>* C;
   int64_t lda[2], ldb[2], ldc;
   int m, n, k[2];
-  int opA;
-  int tiles_m, tiles_n;
   T alpha, beta;
 };
 
@@ -42,8 +39,17 @@ template <class T> struct SkinnyDesc {
   T beta;
 };
 
+// Most tiles of edge 64 and of edge 32 that any descriptor of a launch has.
+struct GemmTiles {
+  int t64 = 0, t32 = 0;
+  void add(int64_t m, int64_t n) {
+    const int64_t a = ((m + 63) / 64) * ((n + 63) / 64), b = ((m + 31) / 32) * ((n + 31) / 32);
+    if (a > t64) t64 = (int)a;
+    if (b > t32) t32 = (int)b;
+  }
+};
 template <class T>
-hipError_t launch_gemm_batched(const GemmDesc<T>* d_descs, int ndesc, int max_tiles, hipStream_t s);
+hipError_t launch_gemm_batched(const GemmDesc<T>* d_descs, int ndesc, GemmTiles t, hipStream_t s);
 template <class T>
 // nmin / nmax: smallest / largest block size in the list; blocks of 96..512
 // rows take the multi-workgroup form (panel kernel + tiled MFMA update).

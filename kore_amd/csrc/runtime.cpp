@@ -579,9 +579,11 @@ template <class T> struct Level {
   InvDesc<T>* inv = nullptr;
   int ninv = 0, maxn_inv = 0, minn_inv = 1 << 30;
   GemmDesc<T>* g1 = nullptr;
-  int ng1 = 0, t1 = 0;
+  int ng1 = 0;
+  GemmTiles t1;
   GemmDesc<T>* g2 = nullptr;
-  int ng2 = 0, t2 = 0;
+  int ng2 = 0;
+  GemmTiles t2;
   SkinnyDesc<T>* fw = nullptr;
   int nfw = 0, mfw = 0;
   SkinnyDesc<T>* fy = nullptr;          // lean form: y_odd = Dinv_odd b_odd before fw
@@ -621,7 +623,8 @@ template <class T> struct Factor : FactorBase {
   bool tail = false;
   GemmDesc<T>* tail1 = nullptr;     // P and R
   GemmDesc<T>* tail2 = nullptr;     // Q
-  int tail_tiles1 = 0, tail_tiles2 = 0, tail_m = 0;
+  GemmTiles tail_tiles1, tail_tiles2;
+  int tail_m = 0;
   SkinnyDesc<T>* tail_solve = nullptr;   // two descriptors
   // Level 0 of a sweep with one right-hand side and an FP64 factor (at least
   // two levels before the tail): its couplings L, U are the sparse
@@ -866,14 +869,12 @@ template <class T> static int32_t factor_build(kore_sys* s, Factor<T>* F) {
   std::vector<Rng> rinv(nlev + 1), rg1(nlev), rg2(nlev), rfw(nlev), rbw(nlev), rfy(nlev, Rng{0, 0});
   F->lev.resize(nlev);
   double flops = 0;
-  auto tiles = [](int m, int n) { return ((m + 63) / 64) * ((n + 63) / 64); };
   auto mkgemm = [&](cx<T>* C, int m, int n, const cx<T>* A1, const cx<T>* B1, int k1, int lda1, int ldb1,
                     const cx<T>* A2, const cx<T>* B2, int k2, int lda2, int ldb2, T alpha, T beta) {
     GemmDesc<T> g{};
     g.A[0] = A1; g.B[0] = B1; g.k[0] = A1 ? k1 : 0; g.lda[0] = lda1; g.ldb[0] = ldb1;
     g.A[1] = A2; g.B[1] = B2; g.k[1] = A2 ? k2 : 0; g.lda[1] = lda2; g.ldb[1] = ldb2;
-    g.C = C; g.ldc = m; g.m = m; g.n = n; g.opA = 0;
-    g.tiles_m = (m + 63) / 64; g.tiles_n = (n + 63) / 64;
+    g.C = C; g.ldc = m; g.m = m; g.n = n;
     g.alpha = alpha; g.beta = beta;
     flops += 8.0 * m * n * ((A1 ? k1 : 0) + (A2 ? k2 : 0));
     F->flops_gemm += 8.0 * m * n * ((A1 ? k1 : 0) + (A2 ? k2 : 0));
@@ -1015,12 +1016,12 @@ template <class T> static int32_t factor_build(kore_sys* s, Factor<T>* F) {
         const int kp = id[t - 1];
         vg.push_back(mkgemm(F->G[k], m, (int)nk(kp), F->D[k], Lp(l, t), m, m, m, nullptr, nullptr, 0, 0, 0, T(1),
                             T(0)));
-        L.t1 = std::max(L.t1, tiles(m, (int)nk(kp)));
+        L.t1.add(m, (int)nk(kp));
         if (t + 1 <= T_ - 1) {
           const int kn = id[t + 1];
           vg.push_back(mkgemm(F->H[k], m, (int)nk(kn), F->D[k], Up(l, t), m, m, m, nullptr, nullptr, 0, 0, 0, T(1),
                               T(0)));
-          L.t1 = std::max(L.t1, tiles(m, (int)nk(kn)));
+          L.t1.add(m, (int)nk(kn));
         }
       }
       if (l == nlev - 1) {
@@ -1029,7 +1030,7 @@ template <class T> static int32_t factor_build(kore_sys* s, Factor<T>* F) {
         const int k0 = id[0], k1 = id[1];
         const int n0 = (int)nk(k0), n1 = (int)nk(k1);
         vg.push_back(mkgemm(F->H[k0], n0, n1, Up(l, 0), F->D[k1], n1, n0, n1, nullptr, nullptr, 0, 0, 0, T(1), T(0)));
-        L.t1 = std::max(L.t1, tiles(n0, n1));
+        L.t1.add(n0, n1);
       }
       rg1[l].n = vg.size() - rg1[l].off;
       rg2[l].off = vg.size();
@@ -1043,19 +1044,19 @@ template <class T> static int32_t factor_build(kore_sys* s, Factor<T>* F) {
                               hasE ? (int)nk(kp) : 0, m, hasE ? (int)nk(kp) : 0, hasF ? Up(l, t) : nullptr,
                               hasF ? F->G[kn] : nullptr, hasF ? (int)nk(kn) : 0, m, hasF ? (int)nk(kn) : 0, T(-1),
                               T(1)));
-          L.t2 = std::max(L.t2, tiles(m, m));
+          L.t2.add(m, m);
         }
         if (t - 2 >= 0) {
           const int kp = id[t - 1], kpp = id[t - 2];
           vg.push_back(mkgemm(Lp(l + 1, t / 2), m, (int)nk(kpp), Lp(l, t), F->G[kp], (int)nk(kp), m, (int)nk(kp),
                               nullptr, nullptr, 0, 0, 0, T(-1), T(0)));
-          L.t2 = std::max(L.t2, tiles(m, (int)nk(kpp)));
+          L.t2.add(m, (int)nk(kpp));
         }
         if (t + 2 <= T_ - 1) {
           const int kn = id[t + 1], knn = id[t + 2];
           vg.push_back(mkgemm(Up(l + 1, t / 2), m, (int)nk(knn), Up(l, t), F->H[kn], (int)nk(kn), m, (int)nk(kn),
                               nullptr, nullptr, 0, 0, 0, T(-1), T(0)));
-          L.t2 = std::max(L.t2, tiles(m, (int)nk(knn)));
+          L.t2.add(m, (int)nk(knn));
         }
       }
       rg2[l].n = vg.size() - rg2[l].off;
@@ -1106,13 +1107,13 @@ template <class T> static int32_t factor_build(kore_sys* s, Factor<T>* F) {
         const int kp = id[t - 1];
         vg.push_back(mkgemm(base + P.offE[l][t], m, (int)nk(kp), F->L[k], F->D[kp], (int)nk(kp), m, (int)nk(kp),
                             nullptr, nullptr, 0, 0, 0, T(1), T(0)));
-        L.t1 = std::max(L.t1, tiles(m, (int)nk(kp)));
+        L.t1.add(m, (int)nk(kp));
       }
       if (t + 1 <= T_ - 1) {
         const int kn = id[t + 1];
         vg.push_back(mkgemm(base + P.offF[l][t], m, (int)nk(kn), F->U[k], F->D[kn], (int)nk(kn), m, (int)nk(kn),
                             nullptr, nullptr, 0, 0, 0, T(1), T(0)));
-        L.t1 = std::max(L.t1, tiles(m, (int)nk(kn)));
+        L.t1.add(m, (int)nk(kn));
       }
     }
     // G_t = Dinv_t L_t, H_t = Dinv_t U_t for the eliminated blocks (fused backward solve)
@@ -1122,12 +1123,12 @@ template <class T> static int32_t factor_build(kore_sys* s, Factor<T>* F) {
       const int kp = id[t - 1];
       vg.push_back(mkgemm(F->G[k], m, (int)nk(kp), F->D[k], F->L[k], m, m, m, nullptr, nullptr, 0, 0, 0, T(1),
                           T(0)));
-      L.t1 = std::max(L.t1, tiles(m, (int)nk(kp)));
+      L.t1.add(m, (int)nk(kp));
       if (t + 1 <= T_ - 1) {
         const int kn = id[t + 1];
         vg.push_back(mkgemm(F->H[k], m, (int)nk(kn), F->D[k], F->U[k], m, m, m, nullptr, nullptr, 0, 0, 0, T(1),
                             T(0)));
-        L.t1 = std::max(L.t1, tiles(m, (int)nk(kn)));
+        L.t1.add(m, (int)nk(kn));
       }
     }
     rg1[l].n = vg.size() - rg1[l].off;
@@ -1143,19 +1144,19 @@ template <class T> static int32_t factor_build(kore_sys* s, Factor<T>* F) {
                             hasE ? (int)nk(kp) : 0, m, hasE ? (int)nk(kp) : 0, hasF ? base + P.offF[l][t] : nullptr,
                             hasF ? F->L[kn] : nullptr, hasF ? (int)nk(kn) : 0, m, hasF ? (int)nk(kn) : 0, T(-1),
                             T(1)));
-        L.t2 = std::max(L.t2, tiles(m, m));
+        L.t2.add(m, m);
       }
       if (t - 2 >= 0) {
         const int kp = id[t - 1], kpp = id[t - 2];
         vg.push_back(mkgemm(F->L[k], m, (int)nk(kpp), base + P.offE[l][t], F->L[kp], (int)nk(kp), m, (int)nk(kp),
                             nullptr, nullptr, 0, 0, 0, T(-1), T(0)));
-        L.t2 = std::max(L.t2, tiles(m, (int)nk(kpp)));
+        L.t2.add(m, (int)nk(kpp));
       }
       if (t + 2 <= T_ - 1) {
         const int kn = id[t + 1], knn = id[t + 2];
         vg.push_back(mkgemm(F->U[k], m, (int)nk(knn), base + P.offF[l][t], F->U[kn], (int)nk(kn), m, (int)nk(kn),
                             nullptr, nullptr, 0, 0, 0, T(-1), T(0)));
-        L.t2 = std::max(L.t2, tiles(m, (int)nk(knn)));
+        L.t2.add(m, (int)nk(knn));
       }
     }
     rg2[l].n = vg.size() - rg2[l].off;
@@ -1216,8 +1217,9 @@ template <class T> static int32_t factor_build(kore_sys* s, Factor<T>* F) {
     vg.push_back(mkgemm(F->H[k1], n1, n0, F->G[k1], F->D[k0], n0, n1, n0, nullptr, nullptr, 0, 0, 0, T(1), T(0)));
     rtail2 = vg.size();
     vg.push_back(mkgemm(F->D[k1], n1, n1, F->G[k1], F->G[k0], n0, n1, n0, nullptr, nullptr, 0, 0, 0, T(1), T(1)));
-    F->tail_tiles1 = std::max(tiles(n0, n1), tiles(n1, n0));
-    F->tail_tiles2 = tiles(n1, n1);
+    F->tail_tiles1.add(n0, n1);
+    F->tail_tiles1.add(n1, n0);
+    F->tail_tiles2.add(n1, n1);
     F->tail_m = std::max(n0, n1);
     const double sb = F->solve_bytes;      // the replaced launches already counted these bytes
     rtails = vs.size();
@@ -2987,13 +2989,14 @@ static int32_t ws_gemm_dev(kore_ws* w, int d0, int nd, int s0, int ns, const cx<
   g.B[0] = Q; g.ldb[0] = ldq;
   g.k[0] = ns;
   g.C = wcol(w, d0); g.ldc = n;
-  g.m = (int)n; g.n = nd; g.opA = 0;
-  g.tiles_m = (int)((n + 63) / 64); g.tiles_n = (nd + 63) / 64;
+  g.m = (int)n; g.n = nd;
   g.alpha = alpha; g.beta = beta;
+  GemmTiles t;
+  t.add(n, nd);
   GemmDesc<double>* dd = w->descb.as<GemmDesc<double>>() + DOT_MAXCHUNK + 1;
   TRY(w->up.put(dd, &g, sizeof(g)));
   Timed tm(c, KORE_TIMER_ORTHO);
-  HIP_TRY(launch_gemm_batched<double>(dd, 1, std::min(g.tiles_m * g.tiles_n, 65535), c->stream));
+  HIP_TRY(launch_gemm_batched<double>(dd, 1, t, c->stream));
   return KORE_OK;
 }
 

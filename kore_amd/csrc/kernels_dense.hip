@@ -8,6 +8,8 @@
 //                  updates on MFMA.
 //
 // All blocks are column-major with interleaved complex storage.
+#include <climits>
+#include <type_traits>
 #include "kore_device.hpp"
 #include "kore_kernels.hpp"
 
@@ -42,9 +44,11 @@ template <class T> __device__ __forceinline__ cx<T> gld_at(const cx<T>* base, un
 // threads).  A and B tiles wholly or partly outside the matrices read their
 // last row or column instead (rows and columns of C that are not stored), so
 // that only the last slab of a product has anything to check: its missing k
-// count as zero.
+// count as zero.  With roles given, rows of C whose role is rmin or more are
+// replaced (their old values count as zero).
 template <class T, int S>
-__device__ __forceinline__ void gemm_tile_body(const GemmDesc<T>& d, const int tile, GemmLds<T, S>& sm) {
+__device__ __forceinline__ void gemm_tile_body(const GemmDesc<T>& d, const int tile, GemmLds<T, S>& sm,
+                                               const int* roles = nullptr, int rmin = 0) {
   using A4 = typename acc4<T>::type;
   constexpr int TS = 32 * S, NQ = 2 * S;      // tile edge, slab elements of A (and of B) per thread
   constexpr int NBUF = GT_NBUF<T>;
@@ -200,13 +204,14 @@ __device__ __forceinline__ void gemm_tile_body(const GemmDesc<T>& d, const int t
   for (int rs = 0; rs < S; ++rs) {
     const int gi = i0 + wr + 16 * rs + l16;
     cx<T> o[S][4];
+    const bool old = acc && gi < d.m && !(roles && roles[gi] >= rmin);
 #pragma unroll
     for (int cs = 0; cs < S; ++cs)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int gj = j0 + wc + 16 * cs + mfma_mrow<T>(lq, r);
         o[cs][r] = czero<T>();
-        if (acc && gi < d.m && gj < d.n) o[cs][r] = gld(d.C + (int64_t)gj * d.ldc + gi);
+        if (old && gj < d.n) o[cs][r] = gld(d.C + (int64_t)gj * d.ldc + gi);
       }
 #pragma unroll
     for (int cs = 0; cs < S; ++cs)
@@ -561,7 +566,7 @@ __global__ __launch_bounds__(512) void gj_inverse_kernel(const InvDesc<T>* __res
 // one compute unit: per panel J = [p0, p0+w)
 //   gj_panel_kernel   one workgroup per block: Gauss-Jordan on the panel
 //                     columns in registers (pivot rows P), C -> M[:, J],
-//                     R = M[P, :] (rows before the update, zero on J) -> scratch;
+//                     R = M[P, :] (rows before the update) -> scratch;
 //   gj_update_kernel  M[i, j] <- [i not in P] M[i, j] + sum_k C[i, k] R[k, j]
 //                     for j outside J, on matrix cores;
 // then gj_perm_kernel twice: A^{-1}[k, l] = M[r_k, r^{-1}(l)] through the
@@ -572,16 +577,6 @@ __global__ __launch_bounds__(512) void gj_inverse_kernel(const InvDesc<T>* __res
 // transforms, T differs from the identity only in the pivot columns P, so for
 // a column j outside J,  T M[:, j] = [i not in P] M[i, j] + T[:, P] M[P, j],
 // and T[:, P] is exactly what in-place elimination leaves in M[:, J].
-// v[idx] by selects, so a register array never becomes indexable memory
-template <int N, class V>
-__device__ __forceinline__ V pick(const V (&v)[N], int idx) {
-  V x = v[0];
-#pragma unroll
-  for (int q = 1; q < N; ++q)
-    if (q == idx) x = v[q];
-  return x;
-}
-
 constexpr int GJM_WP = 32;
 constexpr int GJ_MULTI_MIN = 96;          // blocks at least this large take the multi-workgroup form
 // Two-level panels for blocks of at least GJ_OUTER_MIN rows: the panels of
@@ -609,27 +604,67 @@ __device__ __forceinline__ void gj_outer_range(int n, int p0, int& q0, int& wo) 
   }
 }
 
-// NT threads, NT / NMAX per row.  A column step is a dependent chain (pivot
-// key, wave and workgroup reductions, pivot-row read, reciprocal) plus the
-// row updates.  Blocks of up to 256 rows: complex128 takes 512 threads, two
-// per row, so that a second wave per SIMD hides the chain's latencies;
-// complex64, whose updates cost half as much, takes 256 threads, one per row
-// (measured at 200-row blocks: 256 threads make the complex64 factorisation
-// 1.6 % faster and the complex128 one 4 % slower).  Larger blocks: 512.
-template <class T>
-constexpr int GJ_PANEL_NT256 = sizeof(T) == 4 ? 256 : 512;
+// MFMA row index -> column of a 16-column tile, so that register i of lane
+// group lq holds column 4 i + lq for both element types (the two instructions
+// number their result rows differently, see mfma_mrow).
+template <class T> __device__ __forceinline__ int gj_tile_col(int m);
+template <> __device__ __forceinline__ int gj_tile_col<double>(int m) { return m; }
+template <> __device__ __forceinline__ int gj_tile_col<float>(int m) { return 4 * (m & 3) + (m >> 2); }
 
-template <class T, int NMAX, int NT>
-__global__ __launch_bounds__(NT) void gj_panel_kernel(const InvDesc<T>* __restrict__ descs, int p0) {
-  constexpr int NW = NT / 64, WP = GJM_WP;
-  constexpr int TPR = NT / NMAX, CPT = WP / TPR;
-  static_assert(TPR >= 1 && CPT * TPR == WP, "panel split");
-  // the pivot row; its two column slices are one complex apart beyond their
-  // natural offset, so that the two slices of a wave's reads fall in
-  // different LDS banks
-  constexpr int SL = CPT + (TPR > 1 ? 1 : 0);
-  __shared__ cx<T> sRow[2][TPR * SL];
-  __shared__ unsigned sKey[2][NW];
+// Magnitude bits of a pivot candidate, of which the key keeps the top 22 below
+// the sign (a double's exponent and 11 mantissa bits, a float's and 14); NaN
+// and infinity count as zero.
+__device__ __forceinline__ unsigned pivot_bits(double mag) {
+  const unsigned b = (unsigned)__double2hiint(mag);
+  return b < 0x7FF00000u ? b : 0u;
+}
+__device__ __forceinline__ unsigned pivot_bits(float mag) {
+  const unsigned b = __float_as_uint(mag);
+  return b < 0x7F800000u ? b : 0u;
+}
+
+// Gauss-Jordan on the panel's columns, TPR threads per row.  The panel's 32
+// columns stay in MFMA accumulators; SW = 8 of them at a time are handed to the
+// rows' threads through LDS and eliminated there, a step updating only those 8
+// columns, and the other columns receive the 8 transforms at once as a product
+// on the matrix cores (the composition used for panels and outer panels, one
+// level down).
+//
+// What bounds it is the chain of a column step: key, two barriers with an LDS
+// exchange each, multiplier, next key.  Its length is instructions issued
+// between those points (about 150 and 1300 clocks a step before, about 100 and
+// 920 (complex64) to 1150 clocks now, 200 rows), so the chain holds only what it
+// must: the pivot row is stored and read with 8 columns instead of 32, each
+// thread forms the reciprocal of its own candidate and updates its other columns
+// behind the key's exchange, the waves' keys meet in one LDS maximum, and a
+// row's use and identity are masks in its key.  The pivot rows of the other
+// columns of the outer panel are gathered while later columns are eliminated
+// (fetched after the last step they took 8 of a panel's 44 us, being scattered).
+// Measured, one panel of one block, us before / now: complex128 200 rows 47 / 32,
+// 500 rows 62 / 48; complex64 200 rows 41 / 27, 500 rows 44 / 36; 256 blocks of 500
+// rows: complex128 101 / 65 per launch.  Two threads a row (a thread then stores
+// and reads four columns) are faster except for complex128 above 256 rows, whose
+// accumulators do not leave room for the second wave (one block of 500 rows: 1100
+// against 1000 us for an inversion).
+constexpr int GJ_SW = 8;
+template <class T, int NMAX> constexpr int GJ_TPR = sizeof(T) == 8 && NMAX > 256 ? 1 : 2;
+// columns of a pivot row that a panel keeps in flight: all of an outer panel's
+constexpr int gj_gather_cols(int nmax) { return nmax <= 256 ? 256 : 128; }
+
+template <class T, int NMAX>
+__global__ __launch_bounds__((NMAX * GJ_TPR<T, NMAX>), (sizeof(T) == 4 ? 4 : 2)) void gj_panel_kernel(
+    const InvDesc<T>* __restrict__ descs, int p0) {
+  using A4 = typename acc4<T>::type;
+  constexpr int SW = GJ_SW, TPR = GJ_TPR<T, NMAX>;
+  constexpr int NT = NMAX * TPR, NW = NT / 64, WP = GJM_WP, NK = SW / 4;
+  constexpr int RW = 64 / TPR, NRT = RW / 16, CPT = SW / TPR;   // rows and row tiles of a wave, columns per thread
+  constexpr int LX = NMAX + (TPR > 1 ? 8 : 0);                  // the two columns of a wave's access in different banks
+  static_assert(WP == 32 && SW == 8, "panel split");
+  __shared__ cx<T> sX[SW * LX];           // eliminated columns, row by row: column k of row r at k LX + r
+  __shared__ cx<T> sR[SW * WP];           // pivot rows before the update
+  __shared__ cx<T> sRow[2][SW];           // the pivot row
+  __shared__ cx<T> sInv[SW];              // minus the inverse pivots
+  __shared__ unsigned sKey[4];            // best key of a step; steps take the four in turn
   __shared__ int sPiv[WP];
   __shared__ int sSing;
   const InvDesc<T> d = descs[blockIdx.x];
@@ -637,149 +672,271 @@ __global__ __launch_bounds__(NT) void gj_panel_kernel(const InvDesc<T>* __restri
   if (p0 >= n) return;                    // uniform: this block is already done
   const int64_t ld = d.ld;
   cx<T>* __restrict__ M = d.M;
-  int* __restrict__ rowof = d.ipiv;
   cx<T>* __restrict__ R = d.scratch;
   int* __restrict__ roles = reinterpret_cast<int*>(d.scratch + (size_t)WP * n);
   const int w = min(WP, n - p0);
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int r = tid / TPR, h = tid % TPR;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int l16 = lane & 15, lq = lane >> 4;
+  const int r = tid / TPR, h = tid % TPR;   // owned row, columns [CPT h, CPT h + CPT) of the SW at hand
   const bool live = r < n;
-  if (tid == 0) sSing = 0;
-  for (int q = tid; q < WP; q += NT) sPiv[q] = 0;
-  __syncthreads();
+  cx<T>* J = M + (int64_t)p0 * ld;        // the panel's columns
+  // row tile rt of the wave, column 16 ct + 4 i + lq
+  A4 cre[NRT][2], cim[NRT][2];
+#pragma unroll
+  for (int rt = 0; rt < NRT; ++rt)
+#pragma unroll
+    for (int ct = 0; ct < 2; ++ct)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int row = RW * wave + 16 * rt + l16, j = 16 * ct + 4 * i + lq;
+        cx<T> x = gld_at<T>(J, (unsigned)min(j, w - 1) * (unsigned)ld + (unsigned)min(row, n - 1));
+        if (row >= n || j >= w) x = czero<T>();
+        cre[rt][ct][i] = x.re;
+        cim[rt][ct][i] = x.im;
+      }
   // every row is unused at the first panel (the scratch holds an earlier call's
   // roles); afterwards a row's role is the column it pivots, or -1
   int role = -2;
   if (live) role = p0 == 0 ? -1 : roles[r];
+  // zero in a vector register that the compiler cannot see through: for an LDS
+  // address that it knows to be the same in all lanes it would reduce over the
+  // lanes once more before an atomic
+  int zero_off = 0;
+  asm("" : "+v"(zero_off));
+  int sing = INT_MAX;                     // smallest singular column (1-based) that this thread has met
+  if (tid == 0) sSing = INT_MAX;
+  if (tid < 4) sKey[tid] = 0;
+  if (tid < WP) sPiv[tid] = 0;
+  __syncthreads();
   int q0, wo;
   gj_outer_range(n, p0, q0, wo);
-  cx<T> myipv = czero<T>();               // this row's inverse pivot, if it becomes a pivot row
-  cx<T> v[CPT];
+  // R[k, j] = M[P[k], j] for the columns j of the outer panel (those of the panel
+  // itself are not used): the rows of SW columns are requested as soon as they
+  // are known and stored after the next SW columns, behind whose steps the
+  // scattered reads finish.  GP passes of GC columns are kept in flight.
+  constexpr int GC = NT / SW, GP = gj_gather_cols(NMAX) / GC;
+  cx<T> gx[GP];
+  const int gk = tid % SW, gj = tid / SW;
+  auto gather = [&](int s0) __attribute__((always_inline)) {
+    const cx<T>* row = M + sPiv[s0 + gk] + (int64_t)q0 * ld;
 #pragma unroll
-  for (int jj = 0; jj < CPT; ++jj) {
-    const int j = h * CPT + jj;
-    v[jj] = (live && j < w) ? M[(int64_t)(p0 + j) * ld + r] : czero<T>();
-  }
-  // one elimination step per panel column; the two half loops keep each
-  // unrolled body small enough that the compiler unrolls it fully, so that v
-  // is indexed by constants only and stays in registers
-  auto step = [&](const int c) {
-    if (c < w) {                          // uniform
-      const int par = c & 1;
-      unsigned key = 0;
-      if (live && h == c / CPT && role == -1) key = pivot_key32((double)cabs1(pick<CPT>(v, c % CPT)), r);
-      key = wave_max_u32(key);
-      if (lane == 0) sKey[par][wave] = key;
-      __syncthreads();
-      // the workgroup's best key by a tree over the waves' keys
-      unsigned kk[NW];
+    for (int t = 0; t < GP; ++t) gx[t] = gld(row + (int64_t)min(gj + t * GC, wo - 1) * ld);
+    for (int j = gj + GP * GC; j < wo; j += GC) gst(R + (int64_t)(q0 + j) * WP + s0 + gk, gld(row + (int64_t)j * ld));
+  };
+  auto put = [&](int s0) __attribute__((always_inline)) {
 #pragma unroll
-      for (int qq = 0; qq < NW; ++qq) kk[qq] = sKey[par][qq];
+    for (int t = 0; t < GP; ++t) {
+      const int j = gj + t * GC;
+      if (j < wo) gst(R + (int64_t)(q0 + j) * WP + s0 + gk, gx[t]);
+    }
+  };
+  auto wave_sync = []() __attribute__((always_inline)) {   // LDS written by this wave's other lanes
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  };
+  // columns [SW s, SW s + SW) between the accumulators and the rows' threads; s
+  // is a compile-time constant here, so that the accumulators are never indexed
+  auto extract = [&](auto sc) __attribute__((always_inline)) {
+    constexpr int S = decltype(sc)::value, CT = S * SW / 16, I0 = (S * SW % 16) / 4;
 #pragma unroll
-      for (int st = 1; st < NW; st *= 2)
+    for (int rt = 0; rt < NRT; ++rt)
 #pragma unroll
-        for (int i = 0; i + st < NW; i += 2 * st) kk[i] = max(kk[i], kk[i + st]);
-      const unsigned best = kk[0];
-      const int p = best ? 511 - (int)(best & 0x1FFu) : 0;
-      if (tid == 0) sPiv[c] = p;
-      if (r == p) role = p0 + c;
-      // only the pivot row's lanes write it, behind a second barrier: one
-      // row of stores per column instead of every wave storing its best
-      // candidate before the keys are compared (measured: a 500-row FP64
-      // panel 102.5 -> 74.7 us for one block, 258 -> 204 us for 300)
-      if (best != 0 && r == p) {
+      for (int k = 0; k < NK; ++k)
+        sX[(4 * k + lq) * LX + RW * wave + 16 * rt + l16] = cx<T>{cre[rt][CT][I0 + k], cim[rt][CT][I0 + k]};
+  };
+  auto update = [&](auto sc, int kw) __attribute__((always_inline)) {
+    constexpr int S = decltype(sc)::value, CT = S * SW / 16, I0 = (S * SW % 16) / 4;
+    cx<T> b[2][NK];
 #pragma unroll
-        for (int jj = 0; jj < CPT; ++jj) sRow[par][h * SL + jj] = v[jj];
+    for (int ct = 0; ct < 2; ++ct)
+#pragma unroll
+      for (int k = 0; k < NK; ++k) {
+        b[ct][k] = sR[(4 * k + lq) * WP + 16 * ct + gj_tile_col<T>(l16)];
+        if (4 * k + lq >= kw) b[ct][k] = czero<T>();
       }
-      __syncthreads();
-      const cx<T>* __restrict__ prow = sRow[par];
-      cx<T> pv = prow[(c / CPT) * SL + c % CPT];
-      T den = pv.re * pv.re + pv.im * pv.im;
-      if (!(den > T(0))) {
-        if (tid == 0 && sSing == 0) sSing = p0 + c + 1;
-        pv = cx<T>{tiny_pivot<T>(), T(0)};
-        den = pv.re * pv.re;
-      }
-      const T iden = T(1) / den;
-      const cx<T> ipv{pv.re * iden, -pv.im * iden};
-      cx<T> vc = pick<CPT>(v, c % CPT);
-      if constexpr (TPR == 2) {
-        if (c / CPT == 0) {
-          vc.re = dpp_t<0xA0>(vc.re);
-          vc.im = dpp_t<0xA0>(vc.im);
-        } else {
-          vc.re = dpp_t<0xF5>(vc.re);
-          vc.im = dpp_t<0xF5>(vc.im);
-        }
-      }
-      // Rows past n and columns past w hold zeros (and the pivot row's copy
-      // too), so the update needs no row or column guard: zeros stay zeros.
-      // Column c is held by slice c / CPT at register c % CPT.
-      // The pivot row is not scaled here: its column c becomes 1 and the row
-      // is multiplied by its inverse pivot once, after the panel (a later
-      // step updates it like any other row, which commutes with that scale).
-      // So every lane runs the same code, the pivot row with multiplier zero.
-      const bool isp = r == p;
-      if (isp) myipv = ipv;
-      cx<T> l = cmul(vc, ipv);
-      if (isp) l = czero<T>();
-      const cx<T> nl{-l.re, -l.im}, sc = isp ? cx<T>{T(1), T(0)} : nl;
 #pragma unroll
-      for (int jj = 0; jj < CPT; ++jj) {
-        const cx<T> u = prow[h * SL + jj];
-        v[jj] = (jj == c % CPT && h == c / CPT) ? sc : cfma(v[jj], nl, u);   // four FMAs
+    for (int rt = 0; rt < NRT; ++rt) {
+      cx<T> a[NK];
+#pragma unroll
+      for (int k = 0; k < NK; ++k) a[k] = sX[(4 * k + lq) * LX + RW * wave + 16 * rt + l16];
+#pragma unroll
+      for (int ct = 0; ct < 2; ++ct)
+#pragma unroll
+        for (int k = 0; k < NK; ++k) cmma<T>(cre[rt][ct], cim[rt][ct], a[k], b[ct][k]);
+#pragma unroll
+      for (int k = 0; k < NK; ++k) {
+        cre[rt][CT][I0 + k] = a[k].re;
+        cim[rt][CT][I0 + k] = a[k].im;
       }
     }
   };
+  auto eliminate = [&](auto sc) __attribute__((always_inline)) {
+    constexpr int s0 = decltype(sc)::value * SW;
+    const int kw = min(SW, w - s0);
+    if (kw <= 0) return;                  // uniform
+    extract(sc);
+    wave_sync();
+    cx<T> v[CPT];
 #pragma unroll
-  for (int c = 0; c < WP / 2; ++c) step(c);
+    for (int k = 0; k < CPT; ++k) v[k] = sX[(CPT * h + k) * LX + r];
+    // A step's key is one mask and one or: rows in use have both zero.  Every
+    // column has an unused row left, so the best key is never zero.
+    const unsigned rowkey = 0x80000000u | (unsigned)(511 - r);
+    unsigned rk = role == -1 && h == 0 ? rowkey : 0u, mk = role == -1 && h == 0 ? 0x7FFFFE00u : 0u;
+    unsigned mykey = 0;                   // of the row (of both its lanes)
+    // the row's entry x of column s0 + c enters the search for its pivot
+    auto compete = [&](cx<T> x, int c) __attribute__((always_inline)) {
+      mykey = (pivot_bits(cabs1(x)) & mk) | rk;
+      unsigned key = mykey;
+      key = max(key, dpp_u32<0xB1>(key));  // quad_perm [1,0,3,2]
+      if constexpr (TPR == 2) mykey = key;
+      key = max(key, dpp_u32<0x4E>(key));  // quad_perm [2,3,0,1]
+      key = max(key, dpp_u32<0x141>(key)); // row_half_mirror
+      key = max(key, dpp_u32<0x140>(key)); // row_mirror
+      if (l16 == 15) __hip_atomic_fetch_max(&sKey[zero_off + (c & 3)], key, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    };
+    // minus its reciprocal, should it win
+    bool zero = false;
+    auto invert = [&](cx<T> x) __attribute__((always_inline)) {
+      T den = x.re * x.re + x.im * x.im;
+      zero = !(den > T(0));
+      if (zero) {
+        x = cx<T>{tiny_pivot<T>(), T(0)};
+        den = x.re * x.re;
+      }
+      const T iden = T(1) / den;
+      return cx<T>{-(x.re * iden), x.im * iden};
+    };
+    compete(v[0], s0);
+    cx<T> ninv = invert(v[0]);
 #pragma unroll
-  for (int c = WP / 2; c < WP; ++c) step(c);
-  if (role >= p0) {                       // pivot rows of this panel: the deferred scale
+    for (int c = 0; c < SW; ++c) {
+      if (c < kw) {                       // uniform
+        const int hc = c / CPT, vc = c % CPT;   // where column c is
+        __syncthreads();
+        const bool isp = sKey[(s0 + c) & 3] == mykey;
+        // only the pivot row's threads store it, behind a second barrier (every
+        // wave storing its best candidate beside its key costs more)
+        if (isp) {
 #pragma unroll
-    for (int jj = 0; jj < CPT; ++jj) v[jj] = cmul(v[jj], myipv);
-  }
-  __syncthreads();
-  // C -> M[:, J]; R = M[P, :] on the outer panel's columns outside J, and
-  // those entries of M cleared (disjoint columns, so the order of the two
-  // does not matter; the update kernel has not run yet): the update adds
-  // C R to every row, which replaces the pivot rows and accumulates into the
-  // others
-  if (live) {
+          for (int k = 0; k < CPT; ++k) sRow[c & 1][CPT * h + k] = v[k];
+          if (h == hc) {
+            sInv[c] = ninv;
+            if (zero) sing = min(sing, p0 + s0 + c + 1);
+          }
+          role = p0 + s0 + c;
+          rk = mk = 0;
+        }
+        __syncthreads();
+        const cx<T> pinv = sInv[c];
+        cx<T> u[CPT];
 #pragma unroll
-    for (int jj = 0; jj < CPT; ++jj) {
-      const int j = h * CPT + jj;
-      if (j < w) M[(int64_t)(p0 + j) * ld + r] = v[jj];
-    }
-    if (h == 0) roles[r] = role;
-  }
-  if (tid < w) rowof[p0 + tid] = sPiv[tid];
-  constexpr int RB = 8;                   // loads in flight per thread
-  for (int base = 0; base < WP * wo; base += RB * NT) {
-    cx<T> x[RB];
+        for (int k = 0; k < CPT; ++k) u[k] = sRow[c & 1][CPT * h + k];
+        cx<T> x = v[vc];
+        if constexpr (TPR == 2) {         // the row's entry in column c, from the lane that holds it
+          if (hc == 0) {
+            x.re = dpp_t<0xA0>(x.re);     // quad_perm [0,0,2,2]
+            x.im = dpp_t<0xA0>(x.im);
+          } else {
+            x.re = dpp_t<0xF5>(x.re);     // quad_perm [1,1,3,3]
+            x.im = dpp_t<0xF5>(x.im);
+          }
+        }
+        // Rows past n and columns past w hold zeros (and the pivot row's copy
+        // too), so the update needs no row or column guard: zeros stay zeros.
+        // The pivot row is not scaled here: its column c becomes 1 and the row
+        // is multiplied by its inverse pivot once, after the last step (a later
+        // step updates it like any other row, which commutes with that scale).
+        // So every lane runs the same code, the pivot row with multiplier zero.
+        cx<T> nl = cmul(x, pinv);
+        if (isp) nl = czero<T>();
+        const cx<T> fin{isp ? T(1) : nl.re, nl.im};
+        // the next pivot column first: its key is the next link of the chain,
+        // and the other columns' updates and the reciprocal run behind it
+        const int hn = (c + 1) / CPT, vn = (c + 1) % CPT;
+        if (c + 1 < SW) {
+          const cx<T> t = cfma(v[vn], nl, u[vn]);
+          v[vn] = vn == vc && h == hc ? fin : t;
+          if (TPR == 2 && vn == 0) {      // the columns of the other lane slice begin
+            rk = role == -1 && h == hn ? rowkey : 0u;
+            mk = role == -1 && h == hn ? 0x7FFFFE00u : 0u;
+          }
+          if (c + 1 < kw) compete(v[vn], s0 + c + 1);
+        }
+        if (tid == 0) sKey[(s0 + c + 2) & 3] = 0;      // last read two steps ago, next written in the next step
 #pragma unroll
-    for (int t = 0; t < RB; ++t) {
-      const int idx = base + t * NT + tid;
-      const int k = idx % WP, j = q0 + idx / WP;
-      x[t] = czero<T>();
-      if (idx < WP * wo && k < w && (j < p0 || j >= p0 + w)) {
-        cx<T>* p = M + (int64_t)j * ld + sPiv[k];
-        x[t] = *p;
-        *p = czero<T>();                  // the update then replaces the pivot rows
+        for (int k = 0; k < CPT; ++k)
+          if (k != vn || c + 1 == SW) {
+            const cx<T> t = cfma(v[k], nl, u[k]);
+            v[k] = k == vc && h == hc ? fin : t;
+          }
+        if (c + 1 < SW) ninv = invert(v[vn]);
       }
     }
+    const int kp = role >= p0 + s0 ? role - (p0 + s0) : -1;   // pivot row of these columns: which one
+    if (kp >= 0) {                        // the deferred scale
+      const cx<T> ip{-sInv[kp].re, -sInv[kp].im};
+      if (h == 0) sPiv[s0 + kp] = r;
 #pragma unroll
-    for (int t = 0; t < RB; ++t) {
-      const int idx = base + t * NT + tid;
-      if (idx < WP * wo) R[(int64_t)q0 * WP + idx] = x[t];
+      for (int k = 0; k < CPT; ++k) v[k] = cmul(v[k], ip);
+    }
+#pragma unroll
+    for (int k = 0; k < CPT; ++k) sX[(CPT * h + k) * LX + r] = v[k];
+    // the pivot rows' other columns go to sR and are cleared: the product then
+    // replaces the pivot rows and accumulates into the others (what it leaves in
+    // these SW columns is overwritten by their final values)
+#pragma unroll
+    for (int rt = 0; rt < NRT; ++rt) {
+      const int kr = __shfl(kp, (16 * rt + l16) * TPR, 64);
+      if (kr >= 0) {
+#pragma unroll
+        for (int ct = 0; ct < 2; ++ct)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            sR[kr * WP + 16 * ct + 4 * i + lq] = cx<T>{cre[rt][ct][i], cim[rt][ct][i]};
+            cre[rt][ct][i] = T(0);
+            cim[rt][ct][i] = T(0);
+          }
+      }
+    }
+    __syncthreads();
+    if (s0) put(s0 - SW);
+    gather(s0);
+    update(sc, kw);
+  };
+  eliminate(std::integral_constant<int, 0>{});
+  eliminate(std::integral_constant<int, 1>{});
+  eliminate(std::integral_constant<int, 2>{});
+  eliminate(std::integral_constant<int, 3>{});
+  put((w - 1) / SW * SW);
+  // C -> M[:, J]
+#pragma unroll
+  for (int rt = 0; rt < NRT; ++rt) {
+    const int row = RW * wave + 16 * rt + l16;
+    if (row < n) {
+#pragma unroll
+      for (int ct = 0; ct < 2; ++ct)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int j = 16 * ct + 4 * i + lq;
+          if (j < w) gst(J + (int64_t)j * ld + row, cx<T>{cre[rt][ct][i], cim[rt][ct][i]});
+        }
     }
   }
+  if (live && h == 0) roles[r] = role;
+  if (tid < w) d.ipiv[p0 + tid] = sPiv[tid];
   // info: reset by the first panel, then the first singular column wins
-  if (tid == 0 && d.info && (p0 == 0 || (sSing && *d.info == 0))) *d.info = sSing;
+  if (sing != INT_MAX) atomicMin(&sSing, sing);
+  __syncthreads();
+  if (tid == 0 && d.info) {
+    const int col = sSing == INT_MAX ? 0 : sSing;
+    if (p0 == 0 || (col && *d.info == 0)) *d.info = col;
+  }
 }
 
 // The panel's update: M[:, j] += M[:, J] R[:, j] for the columns j of its
-// outer panel outside J (pivot rows cleared by the panel kernel), on the
+// outer panel outside J, the pivot rows' old values counting as zero, on the
 // batched GEMM's tile with descriptors made here (columns [q0, p0), then
 // [p0 + w, q0 + wo)); K = w <= 32.
 template <class T, int S>
@@ -820,7 +977,7 @@ __global__ __launch_bounds__(256, 3) void gj_update_kernel(const InvDesc<T>* __r
   d.n = ncols;
   d.alpha = T(1);
   d.beta = T(1);
-  gemm_tile_body<T, S>(d, t, sm);
+  gemm_tile_body<T, S>(d, t, sm, reinterpret_cast<const int*>(v.scratch + (size_t)GJM_WP * n), p0);
 }
 
 // phase 0: S[l n + k] = M[r_k, r^{-1}(l)];  phase 1: M <- S.   Grid: (column chunks, blocks).
@@ -860,9 +1017,7 @@ __global__ __launch_bounds__(256) void gj_perm_kernel(const InvDesc<T>* __restri
 }
 
 // End of outer panel O = [q0, q0 + wo): R_O[k, j] = M[P_O[k], j] for the
-// columns j outside O (at R_O[j GJ_WO + k]), and those entries of M are
-// cleared (the outer product then adds T_O[:, P_O] R_O to every row, which
-// replaces the pivot rows and accumulates into the others).
+// columns j outside O (at R_O[j GJ_WO + k]).
 template <class T>
 __global__ __launch_bounds__(256) void gj_outer_gather_kernel(const InvDesc<T>* __restrict__ descs, int q0) {
   const InvDesc<T> d = descs[blockIdx.y];
@@ -878,17 +1033,13 @@ __global__ __launch_bounds__(256) void gj_outer_gather_kernel(const InvDesc<T>* 
     const int k = idx % GJ_WO, jc = idx / GJ_WO;
     const int j = jc < q0 ? jc : jc + wo;
     cx<T> x = czero<T>();
-    if (k < wo) {
-      cx<T>* p = M + (int64_t)j * ld + piv[k];
-      x = *p;
-      *p = czero<T>();
-    }
+    if (k < wo) x = gld(M + (int64_t)j * ld + piv[k]);
     RO[(int64_t)j * GJ_WO + k] = x;
   }
 }
 
-// M[:, j] += M[:, O] R_O[:, j] for the columns outside O: the batched GEMM's
-// tile on descriptors made here (columns [0, q0), then [q0 + wo, n)).
+// M[:, j] += M[:, O] R_O[:, j] for the columns outside O, the rows P_O replaced:
+// the batched GEMM's tile on descriptors made here (columns [0, q0), then [q0 + wo, n)).
 template <class T, int S>
 __global__ __launch_bounds__(256, 3) void gj_outer_update_kernel(const InvDesc<T>* __restrict__ descs, int ndesc,
                                                                  int per, int q0) {
@@ -925,7 +1076,7 @@ __global__ __launch_bounds__(256, 3) void gj_outer_update_kernel(const InvDesc<T
   d.n = ncols;
   d.alpha = T(1);
   d.beta = T(1);
-  gemm_tile_body<T, S>(d, t, sm);
+  gemm_tile_body<T, S>(d, t, sm, reinterpret_cast<const int*>(v.scratch + (size_t)GJM_WP * n), q0);
 }
 
 template <class T, int S>
@@ -952,10 +1103,9 @@ static hipError_t launch_gj_inverse_multi(const InvDesc<T>* d_descs, int ndesc, 
   const int nt = (nmax + 63) / 64;
   for (int p0 = 0; p0 < nmax; p0 += GJM_WP) {
     if (nmax <= 256)
-      hipLaunchKernelGGL((gj_panel_kernel<T, 256, GJ_PANEL_NT256<T>>), dim3(ndesc), dim3(GJ_PANEL_NT256<T>), 0, s,
-                         d_descs, p0);
+      hipLaunchKernelGGL((gj_panel_kernel<T, 256>), dim3(ndesc), dim3(256 * GJ_TPR<T, 256>), 0, s, d_descs, p0);
     else
-      hipLaunchKernelGGL((gj_panel_kernel<T, 512, 512>), dim3(ndesc), dim3(512), 0, s, d_descs, p0);
+      hipLaunchKernelGGL((gj_panel_kernel<T, 512>), dim3(ndesc), dim3(512 * GJ_TPR<T, 512>), 0, s, d_descs, p0);
     // the columns an update covers come in multiples of 32 (a panel's width)
     launch_gj_updates<T, 1>(d_descs, ndesc, nmax, p0, s);
     // the end of an outer panel (of every block whose outer panel holds p0)

@@ -3,9 +3,7 @@
 //   gemm_batched   C = beta*C + alpha*(A1*B1 + A2*B2) for a list of complex
 //                  blocks, on MFMA (f64 16x16x4 or f32 16x16x4).
 //   gj_inverse     in-place inverse of a list of complex blocks by blocked
-//                  Gauss-Jordan elimination with partial (row) pivoting,
-//                  one workgroup per block, panel staged in LDS, the rank-w
-//                  updates on MFMA.
+//                  Gauss-Jordan elimination with partial (row) pivoting.
 //
 // All blocks are column-major with interleaved complex storage.
 #include <climits>
@@ -288,24 +286,29 @@ template <class T> __device__ __forceinline__ T tiny_pivot() { return sizeof(T) 
 // ---------------------------------------------------------------------------
 // batched Gauss-Jordan inverse with partial pivoting
 // ---------------------------------------------------------------------------
-// One workgroup of 512 threads per block.  Rows are never moved: column j is
-// eliminated with pivot row r_j (within a factor 1 - 2^-11 of the largest
-// |re|+|im| among the rows not used yet, first index on ties), so that at the end
-//     A^{-1}[k, l] = M[r_k, r^{-1}(l)],
-// applied once through the caller's scratch block.
-//
-// Panel J = [p0, p0+w) with pivot rows P:
-//   1. Gauss-Jordan on the panel columns over all rows, in registers (each
-//      row owned by TPR adjacent lanes, CPT columns each).  One column costs
-//      two barriers: the pivot is a packed 32-bit magnitude|row key reduced
-//      within each wave by DPP and across the waves through LDS; then the
-//      pivot row's lanes store it for all to read.
-//      Afterwards the panel holds C: rows P hold X = M[P, J]^{-1} (permuted),
-//      the other rows hold -M[i, J] X -- the final columns J of M.
-//   2. R = M[P, :] (old pivot rows) is staged in LDS.
-//   3. Outside J:  M[i, j] <- [i not in P] M[i, j] + sum_k C[i, k] R[k, j]
-//      (matrix cores; C read back from the block, R from LDS).
-// Cross-lane moves within rows of 16 lanes (DPP) and lane reads.
+// Rows are never moved: column j is eliminated with pivot row r_j (within a
+// factor 1 - 2^-11 of the largest |re|+|im| among the rows not used yet, first
+// index on ties), so that at the end
+//     A^{-1}[k, l] = M[r_k, r^{-1}(l)].
+// The update of a block spreads over many workgroups: per panel J = [p0, p0+w)
+//   gj_panel_kernel   one workgroup per block: Gauss-Jordan on the panel
+//                     columns (pivot rows P), C -> M[:, J], the final columns
+//                     J of M; R = M[P, :] (rows before the update) -> scratch;
+//   gj_update_kernel  M[i, j] <- [i not in P] M[i, j] + sum_k C[i, k] R[k, j]
+//                     for j outside J, on matrix cores;
+// then gj_perm_kernel twice: A^{-1}[k, l] = M[r_k, r^{-1}(l)] through the
+// scratch block and back.  Blocks of one panel (up to 32 rows) are complete
+// after gj_panel_kernel, which stores them in their final order: one launch
+// (24 rows, complex128: 55 -> 20 us; a kernel that ran the whole elimination of
+// a block in one workgroup, used below 96 rows, is gone: 74 rows 193 -> 94 us).
+// Scratch layout (per block of more than 32 rows, n x n complex): R
+// (32 x n, R[k, j] at R[j 32 + k]), then n ints of row roles (-1 unused,
+// c >= 0: the pivot row of column c).  The multi-panel composition: with T
+// the product of the panel's elementary transforms, T differs from the identity
+// only in the pivot columns P, so for a column j outside J,
+// T M[:, j] = [i not in P] M[i, j] + T[:, P] M[P, j], and T[:, P] is exactly what
+// in-place elimination leaves in M[:, J].
+// Cross-lane moves within rows of 16 lanes (DPP).
 template <int CTRL> __device__ __forceinline__ unsigned dpp_u32(unsigned x) {
   return (unsigned)__builtin_amdgcn_update_dpp(0, (int)x, CTRL, 0xF, 0xF, false);
 }
@@ -316,269 +319,7 @@ template <int CTRL> __device__ __forceinline__ float dpp_t(float x) {
   return __uint_as_float(dpp_u32<CTRL>(__float_as_uint(x)));
 }
 
-// 32-bit pivot key of the Gauss-Jordan kernels: valid flag (bit 31), the
-// magnitude's exponent and top 11 mantissa bits (bits 30-9), 511 - row.  The
-// chosen pivot is within a factor 1 - 2^-11 of the column's largest entry
-// (threshold partial pivoting; ties go to the lower row); one max per
-// reduction stage instead of a 64-bit compare and two selects.
-__device__ __forceinline__ unsigned pivot_key32(double mag, int r) {
-  if (!(mag <= 1.7976931348623157e308)) mag = 0.0;   // NaN / inf never win
-  const unsigned long long b = (unsigned long long)__double_as_longlong(mag);
-  return 0x80000000u | (((unsigned)(b >> 41) & 0x3FFFFFu) << 9) | (unsigned)(511 - r);
-}
-// Maximum over the wavefront, returned to every lane: quad swaps and row
-// mirrors leave each row of 16 lanes with its maximum, then the four rows
-// are combined through lanes 15, 31, 47 and 63.
-__device__ __forceinline__ unsigned wave_max_u32(unsigned v) {
-  v = max(v, dpp_u32<0xB1>(v));        // quad_perm [1,0,3,2]
-  v = max(v, dpp_u32<0x4E>(v));        // quad_perm [2,3,0,1]
-  v = max(v, dpp_u32<0x141>(v));       // row_half_mirror
-  v = max(v, dpp_u32<0x140>(v));       // row_mirror
-  const unsigned a = max((unsigned)__builtin_amdgcn_readlane((int)v, 15), (unsigned)__builtin_amdgcn_readlane((int)v, 31));
-  const unsigned b = max((unsigned)__builtin_amdgcn_readlane((int)v, 47), (unsigned)__builtin_amdgcn_readlane((int)v, 63));
-  return max(a, b);
-}
-
-
-template <class T, int WP, int NMAX>
-__global__ __launch_bounds__(512) void gj_inverse_kernel(const InvDesc<T>* __restrict__ descs) {
-  using A4 = typename acc4<T>::type;
-  constexpr int NT = 512;
-  constexpr int NW = NT / 64;
-  constexpr int TPR = NT / NMAX;         // threads per row
-  constexpr int CPT = WP / TPR;          // panel columns per thread
-  constexpr int LDR = NMAX + 4;          // R: row k at sR[k*LDR + j]
-  static_assert(TPR >= 1 && CPT * TPR == WP, "panel split");
-  __shared__ cx<T> sR[WP * LDR];
-  __shared__ cx<T> sRow[2][WP];           // the pivot row (double-buffered)
-  __shared__ unsigned sKey[2][NW];
-  __shared__ short sRole[NMAX];          // -1 unused, -2 used earlier, c >= 0: pivot c of this panel
-  __shared__ int sPiv[WP];
-  __shared__ int sSing;
-
-  const InvDesc<T> d = descs[blockIdx.x];
-  const int n = d.n;
-  const int64_t ld = d.ld;
-  cx<T>* __restrict__ M = d.M;
-  int* __restrict__ rowof = d.ipiv;      // r_j: pivot row of column j
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int l16 = lane & 15, lq = lane >> 4;
-  const int r = tid / TPR, h = tid % TPR;   // owned row and column slice
-  const bool live = r < n;
-  int role = -1;                          // register copy of sRole[r]
-  if (tid == 0) sSing = 0;
-  for (int q = tid; q < NMAX; q += NT) sRole[q] = -1;
-
-  for (int p0 = 0; p0 < n; p0 += WP) {
-    const int w = min(WP, n - p0);
-    // 1. panel -> registers
-    cx<T> v[CPT];
-#pragma unroll
-    for (int jj = 0; jj < CPT; ++jj) {
-      const int j = h * CPT + jj;
-      v[jj] = (live && j < w) ? M[(int64_t)(p0 + j) * ld + r] : czero<T>();
-    }
-    // Two barriers per column: every wave publishes its best 32-bit key
-    // (pivot_key32: threshold pivoting within 1 - 2^-11 of the largest
-    // entry); after the first barrier all threads pick the best of the
-    // eight, the pivot row's lanes store it, and after the second barrier
-    // all read it (one row of stores per column instead of one per wave).
-#pragma unroll
-    for (int c = 0; c < WP; ++c) {
-      if (c < w) {                        // uniform
-        const int par = c & 1;
-        unsigned key = 0;
-        if (live && h == c / CPT && role == -1) key = pivot_key32((double)cabs1(v[c % CPT]), r);
-        key = wave_max_u32(key);
-        if (lane == 0) sKey[par][wave] = key;
-        __syncthreads();
-        unsigned kk[NW];
-#pragma unroll
-        for (int qq = 0; qq < NW; ++qq) kk[qq] = sKey[par][qq];
-#pragma unroll
-        for (int st = 1; st < NW; st *= 2)
-#pragma unroll
-          for (int i = 0; i + st < NW; i += 2 * st) kk[i] = max(kk[i], kk[i + st]);
-        const unsigned best = kk[0];
-        // every column has an unused row left, so a valid key always exists
-        const int p = best ? 511 - (int)(best & 0x1FFu) : 0;
-        if (tid == 0) {
-          sRole[p] = (short)c;
-          sPiv[c] = p;
-        }
-        if (r == p) role = c;
-        if (best != 0 && r == p) {
-#pragma unroll
-          for (int jj = 0; jj < CPT; ++jj) sRow[par][h * CPT + jj] = v[jj];
-        }
-        __syncthreads();
-        const cx<T>* __restrict__ prow = sRow[par];
-        cx<T> pv = prow[c];
-        T den = pv.re * pv.re + pv.im * pv.im;
-        if (!(den > T(0))) {
-          if (tid == 0 && sSing == 0) sSing = p0 + c + 1;
-          pv = cx<T>{tiny_pivot<T>(), T(0)};
-          den = pv.re * pv.re;
-        }
-        const T iden = T(1) / den;
-        const cx<T> ipv{pv.re * iden, -pv.im * iden};
-        // this row's entry in column c, held by lane slice c / CPT of the row
-        cx<T> vc = v[c % CPT];
-        if constexpr (TPR == 2) {
-          if (c / CPT == 0) {
-            vc.re = dpp_t<0xA0>(vc.re);   // quad_perm [0,0,2,2]
-            vc.im = dpp_t<0xA0>(vc.im);
-          } else {
-            vc.re = dpp_t<0xF5>(vc.re);   // quad_perm [1,1,3,3]
-            vc.im = dpp_t<0xF5>(vc.im);
-          }
-        }
-        if (live) {
-          if (r == p) {
-#pragma unroll
-            for (int jj = 0; jj < CPT; ++jj) {
-              const int j = h * CPT + jj;
-              v[jj] = (j == c) ? ipv : cmul(v[jj], ipv);
-            }
-          } else {
-            const cx<T> l = cmul(vc, ipv);
-#pragma unroll
-            for (int jj = 0; jj < CPT; ++jj) {
-              const int j = h * CPT + jj;
-              if (j == c) {
-                v[jj] = cx<T>{-l.re, -l.im};
-              } else if (j < w) {
-                const cx<T> u = prow[j];
-                v[jj].re -= l.re * u.re - l.im * u.im;
-                v[jj].im -= l.re * u.im + l.im * u.re;
-              }
-            }
-          }
-        }
-      }
-    }
-    // C -> columns J of the block (final values)
-    if (live) {
-#pragma unroll
-      for (int jj = 0; jj < CPT; ++jj) {
-        const int j = h * CPT + jj;
-        if (j < w) M[(int64_t)(p0 + j) * ld + r] = v[jj];
-      }
-    }
-    if (tid < w) rowof[p0 + tid] = sPiv[tid];
-    // 2. R = M[P, :] outside J (rows k >= w are zero)
-    for (int idx = tid; idx < WP * n; idx += NT) {
-      const int k = idx % WP, j = idx / WP;
-      cx<T> x = czero<T>();
-      if (k < w && (j < p0 || j >= p0 + w)) x = M[(int64_t)j * ld + sPiv[k]];
-      sR[k * LDR + j] = x;
-    }
-    __syncthreads();
-    // 3. rank-w update outside J, one wave per 32-row tile
-    const int ntr = (n + 31) / 32, ntc = (n + 31) / 32;
-    for (int tr = wave; tr < ntr; tr += NW) {
-      const int i0 = tr * 32;
-      cx<T> g[2][WP / 4];
-#pragma unroll
-      for (int rs = 0; rs < 2; ++rs)
-#pragma unroll
-        for (int kk = 0; kk < WP / 4; ++kk) {
-          const int gi = i0 + 16 * rs + l16, gk = 4 * kk + lq;
-          g[rs][kk] = (gi < n && gk < w) ? M[(int64_t)(p0 + gk) * ld + gi] : czero<T>();
-        }
-      int prole[2];
-#pragma unroll
-      for (int rs = 0; rs < 2; ++rs) {
-        const int gi = i0 + 16 * rs + l16;
-        prole[rs] = gi < n ? (int)sRole[gi] : -1;
-      }
-      for (int tc = 0; tc < ntc; ++tc) {
-        const int j0 = tc * 32;
-        if (j0 >= p0 && j0 + 32 <= p0 + w) continue;   // tile inside J: already final
-        A4 cre[2][2], cim[2][2];
-#pragma unroll
-        for (int a = 0; a < 2; ++a)
-#pragma unroll
-          for (int b = 0; b < 2; ++b) {
-            cre[a][b] = A4{0, 0, 0, 0};
-            cim[a][b] = A4{0, 0, 0, 0};
-          }
-#pragma unroll
-        for (int kk = 0; kk < WP / 4; ++kk) {
-          cx<T> b[2];
-#pragma unroll
-          for (int cs = 0; cs < 2; ++cs) {
-            const int gj = j0 + 16 * cs + l16;
-            b[cs] = (gj < n) ? sR[(4 * kk + lq) * LDR + gj] : czero<T>();
-          }
-#pragma unroll
-          for (int rs = 0; rs < 2; ++rs)
-#pragma unroll
-            for (int cs = 0; cs < 2; ++cs) cmma<T>(cre[rs][cs], cim[rs][cs], g[rs][kk], b[cs]);
-        }
-#pragma unroll
-        for (int rs = 0; rs < 2; ++rs)
-#pragma unroll
-          for (int cs = 0; cs < 2; ++cs)
-#pragma unroll
-            for (int rr = 0; rr < 4; ++rr) {
-              const int gi = i0 + 16 * rs + l16;
-              const int gj = j0 + 16 * cs + mfma_mrow<T>(lq, rr);
-              if (gi < n && gj < n && (gj < p0 || gj >= p0 + w)) {
-                cx<T>* cp = M + (int64_t)gj * ld + gi;
-                cx<T> x{cre[rs][cs][rr], cim[rs][cs][rr]};
-                if (!(prole[rs] >= 0)) {
-                  const cx<T> o = *cp;
-                  x.re += o.re;
-                  x.im += o.im;
-                }
-                *cp = x;
-              }
-            }
-      }
-    }
-    __syncthreads();
-    // this panel's pivot rows become "used earlier"
-    if (role >= 0) role = -2;
-    for (int c = tid; c < w; c += NT) sRole[sPiv[c]] = -2;
-  }
-  __syncthreads();
-  // A^{-1}[k, l] = M[r_k, r^{-1}(l)]: permute into the scratch block, copy back
-  int* rinv = reinterpret_cast<int*>(sR);
-  for (int j = tid; j < n; j += NT) rinv[rowof[j]] = j;
-  __syncthreads();
-  cx<T>* __restrict__ S = d.scratch;
-  for (int l = 0; l < n; ++l) {
-    const cx<T>* src = M + (int64_t)rinv[l] * ld;
-    for (int k = tid; k < n; k += NT) S[(int64_t)l * n + k] = src[rowof[k]];
-  }
-  __syncthreads();
-  for (int l = 0; l < n; ++l)
-    for (int k = tid; k < n; k += NT) M[(int64_t)l * ld + k] = S[(int64_t)l * n + k];
-  if (tid == 0 && d.info) *d.info = sSing;
-}
-
-// ---------------------------------------------------------------------------
-// batched Gauss-Jordan inverse, multi-workgroup form (large blocks)
-// ---------------------------------------------------------------------------
-// The same elimination as gj_inverse_kernel, split so that the rank-w update
-// of a block spreads over many workgroups (one 64 x 64 tile each) instead of
-// one compute unit: per panel J = [p0, p0+w)
-//   gj_panel_kernel   one workgroup per block: Gauss-Jordan on the panel
-//                     columns in registers (pivot rows P), C -> M[:, J],
-//                     R = M[P, :] (rows before the update) -> scratch;
-//   gj_update_kernel  M[i, j] <- [i not in P] M[i, j] + sum_k C[i, k] R[k, j]
-//                     for j outside J, on matrix cores;
-// then gj_perm_kernel twice: A^{-1}[k, l] = M[r_k, r^{-1}(l)] through the
-// scratch block and back.  Scratch layout (per block, n x n complex): R
-// (32 x n, R[k, j] at R[j 32 + k]), then n ints of row roles (-1 unused,
-// c >= 0: the pivot row of column c).  The
-// multi-panel composition: with T the product of the panel's elementary
-// transforms, T differs from the identity only in the pivot columns P, so for
-// a column j outside J,  T M[:, j] = [i not in P] M[i, j] + T[:, P] M[P, j],
-// and T[:, P] is exactly what in-place elimination leaves in M[:, J].
 constexpr int GJM_WP = 32;
-constexpr int GJ_MULTI_MIN = 96;          // blocks at least this large take the multi-workgroup form
 // Two-level panels for blocks of at least GJ_OUTER_MIN rows: the panels of
 // 32 columns are grouped into outer panels O of GJ_WO columns.  A panel's
 // rank-32 update is applied to the columns of its outer panel only; once the
@@ -611,9 +352,10 @@ template <class T> __device__ __forceinline__ int gj_tile_col(int m);
 template <> __device__ __forceinline__ int gj_tile_col<double>(int m) { return m; }
 template <> __device__ __forceinline__ int gj_tile_col<float>(int m) { return 4 * (m & 3) + (m >> 2); }
 
-// Magnitude bits of a pivot candidate, of which the key keeps the top 22 below
-// the sign (a double's exponent and 11 mantissa bits, a float's and 14); NaN
-// and infinity count as zero.
+// Magnitude bits of a pivot candidate; NaN and infinity count as zero.  A pivot
+// key is a valid flag (bit 31), the magnitude's next 22 bits (a double's exponent
+// and 11 mantissa bits, a float's and 14) and 511 - row: threshold partial
+// pivoting, ties go to the lower row, and one 32-bit maximum per reduction stage.
 __device__ __forceinline__ unsigned pivot_bits(double mag) {
   const unsigned b = (unsigned)__double2hiint(mag);
   return b < 0x7FF00000u ? b : 0u;
@@ -649,7 +391,7 @@ __device__ __forceinline__ unsigned pivot_bits(float mag) {
 constexpr int GJ_SW = 8;
 template <class T, int NMAX> constexpr int GJ_TPR = sizeof(T) == 8 && NMAX > 256 ? 1 : 2;
 // columns of a pivot row that a panel keeps in flight: all of an outer panel's
-constexpr int gj_gather_cols(int nmax) { return nmax <= 256 ? 256 : 128; }
+constexpr int gj_gather_cols(int nmax) { return nmax <= 256 ? nmax : 128; }
 
 template <class T, int NMAX>
 __global__ __launch_bounds__((NMAX * GJ_TPR<T, NMAX>), (sizeof(T) == 4 ? 4 : 2)) void gj_panel_kernel(
@@ -901,30 +643,35 @@ __global__ __launch_bounds__((NMAX * GJ_TPR<T, NMAX>), (sizeof(T) == 4 ? 4 : 2))
       }
     }
     __syncthreads();
-    if (s0) put(s0 - SW);
-    gather(s0);
+    if (wo > w) {                         // the outer panel has other columns
+      if (s0) put(s0 - SW);
+      gather(s0);
+    }
     update(sc, kw);
   };
   eliminate(std::integral_constant<int, 0>{});
   eliminate(std::integral_constant<int, 1>{});
   eliminate(std::integral_constant<int, 2>{});
   eliminate(std::integral_constant<int, 3>{});
-  put((w - 1) / SW * SW);
-  // C -> M[:, J]
+  if (wo > w) put((w - 1) / SW * SW);
+  // C -> M[:, J]; a block of one panel is then complete and is stored in its
+  // final order, A^{-1}[k, l] = C[r_k, r^{-1}(l)]
+  const bool whole = n <= WP;
 #pragma unroll
   for (int rt = 0; rt < NRT; ++rt) {
     const int row = RW * wave + 16 * rt + l16;
+    const int to = __shfl(role, (16 * rt + l16) * TPR, 64);
     if (row < n) {
 #pragma unroll
       for (int ct = 0; ct < 2; ++ct)
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           const int j = 16 * ct + 4 * i + lq;
-          if (j < w) gst(J + (int64_t)j * ld + row, cx<T>{cre[rt][ct][i], cim[rt][ct][i]});
+          if (j < w) gst(J + (whole ? sPiv[j] * ld + to : j * ld + row), cx<T>{cre[rt][ct][i], cim[rt][ct][i]});
         }
     }
   }
-  if (live && h == 0) roles[r] = role;
+  if (live && h == 0 && !whole) roles[r] = role;
   if (tid < w) d.ipiv[p0 + tid] = sPiv[tid];
   // info: reset by the first panel, then the first singular column wins
   if (sing != INT_MAX) atomicMin(&sSing, sing);
@@ -992,7 +739,7 @@ __global__ __launch_bounds__(256) void gj_perm_kernel(const InvDesc<T>* __restri
   const int n = d.n;
   constexpr int CC = 16;                                   // columns per workgroup
   const int l0 = blockIdx.x * CC;
-  if (l0 >= n) return;
+  if (l0 >= n || n <= GJM_WP) return;                      // blocks of one panel are in order already
   const int64_t ld = d.ld;
   cx<T>* __restrict__ M = d.M;
   cx<T>* __restrict__ S = d.scratch;
@@ -1099,13 +846,18 @@ static void launch_gj_outer_updates(const InvDesc<T>* d_descs, int ndesc, int nm
 }
 
 template <class T>
-static hipError_t launch_gj_inverse_multi(const InvDesc<T>* d_descs, int ndesc, int nmax, hipStream_t s) {
+static hipError_t gj_inverse_launches(const InvDesc<T>* d_descs, int ndesc, int nmax, hipStream_t s) {
   const int nt = (nmax + 63) / 64;
   for (int p0 = 0; p0 < nmax; p0 += GJM_WP) {
-    if (nmax <= 256)
+    if (nmax <= 64)
+      hipLaunchKernelGGL((gj_panel_kernel<T, 64>), dim3(ndesc), dim3(64 * GJ_TPR<T, 64>), 0, s, d_descs, p0);
+    else if (nmax <= 128)
+      hipLaunchKernelGGL((gj_panel_kernel<T, 128>), dim3(ndesc), dim3(128 * GJ_TPR<T, 128>), 0, s, d_descs, p0);
+    else if (nmax <= 256)
       hipLaunchKernelGGL((gj_panel_kernel<T, 256>), dim3(ndesc), dim3(256 * GJ_TPR<T, 256>), 0, s, d_descs, p0);
     else
       hipLaunchKernelGGL((gj_panel_kernel<T, 512>), dim3(ndesc), dim3(512 * GJ_TPR<T, 512>), 0, s, d_descs, p0);
+    if (nmax <= GJM_WP) return hipGetLastError();          // one panel, stored in its final order
     // the columns an update covers come in multiples of 32 (a panel's width)
     launch_gj_updates<T, 1>(d_descs, ndesc, nmax, p0, s);
     // the end of an outer panel (of every block whose outer panel holds p0)
@@ -1142,33 +894,15 @@ hipError_t launch_gemm_batched(const GemmDesc<T>* d_descs, int ndesc, GemmTiles 
 }
 
 template <class T>
-hipError_t launch_gj_inverse(const InvDesc<T>* d_descs, int ndesc, int nmin, int nmax, hipStream_t s) {
+hipError_t launch_gj_inverse(const InvDesc<T>* d_descs, int ndesc, int nmax, hipStream_t s) {
   if (ndesc <= 0) return hipSuccess;
-  // the multi-workgroup form keeps R (32 x n) and the row roles in each block's
-  // n x n scratch, which needs n > 32
-  if (nmax >= GJ_MULTI_MIN && nmax <= 512 && nmin > GJM_WP)
-    return launch_gj_inverse_multi<T>(d_descs, ndesc, nmax, s);
-  if constexpr (sizeof(T) == 8) {
-    if (nmax <= 256)
-      hipLaunchKernelGGL((gj_inverse_kernel<T, 32, 256>), dim3(ndesc), dim3(512), 0, s, d_descs);
-    else if (nmax <= 512)
-      hipLaunchKernelGGL((gj_inverse_kernel<T, 16, 512>), dim3(ndesc), dim3(512), 0, s, d_descs);
-    else
-      return hipErrorInvalidValue;
-  } else {
-    if (nmax <= 256)
-      hipLaunchKernelGGL((gj_inverse_kernel<T, 32, 256>), dim3(ndesc), dim3(512), 0, s, d_descs);
-    else if (nmax <= 512)
-      hipLaunchKernelGGL((gj_inverse_kernel<T, 16, 512>), dim3(ndesc), dim3(512), 0, s, d_descs);
-    else
-      return hipErrorInvalidValue;
-  }
-  return hipGetLastError();
+  if (nmax > 512) return hipErrorInvalidValue;
+  return gj_inverse_launches<T>(d_descs, ndesc, nmax, s);
 }
 
 template hipError_t launch_gemm_batched<double>(const GemmDesc<double>*, int, GemmTiles, hipStream_t);
 template hipError_t launch_gemm_batched<float>(const GemmDesc<float>*, int, GemmTiles, hipStream_t);
-template hipError_t launch_gj_inverse<double>(const InvDesc<double>*, int, int, int, hipStream_t);
-template hipError_t launch_gj_inverse<float>(const InvDesc<float>*, int, int, int, hipStream_t);
+template hipError_t launch_gj_inverse<double>(const InvDesc<double>*, int, int, hipStream_t);
+template hipError_t launch_gj_inverse<float>(const InvDesc<float>*, int, int, hipStream_t);
 
 }  // namespace kore

@@ -577,7 +577,7 @@ struct FactorBase {
 
 template <class T> struct Level {
   InvDesc<T>* inv = nullptr;
-  int ninv = 0, maxn_inv = 0, minn_inv = 1 << 30;
+  int ninv = 0, maxn_inv = 0;
   GemmDesc<T>* g1 = nullptr;
   int ng1 = 0;
   GemmTiles t1;
@@ -958,7 +958,6 @@ template <class T> static int32_t factor_build(kore_sys* s, Factor<T>* F) {
       flops += 8.0 * nk(k) * nk(k) * nk(k);
       F->flops_inv += 8.0 * nk(k) * nk(k) * nk(k);
       L.maxn_inv = std::max(L.maxn_inv, (int)nk(k));
-      L.minn_inv = std::min(L.minn_inv, (int)nk(k));
     }
     rinv[l].n = vinv.size() - rinv[l].off;
     if (l == 0 && sp0) {
@@ -1335,7 +1334,7 @@ template <class T> static int32_t factor_run(kore_sys* s, Factor<T>* F) {
     Level<T>& L = F->lev[l];
     {
       Timed tm(c, KORE_TIMER_INV);
-      HIP_TRY(launch_gj_inverse<T>(L.inv, L.ninv, L.minn_inv, L.maxn_inv, st));
+      HIP_TRY(launch_gj_inverse<T>(L.inv, L.ninv, L.maxn_inv, st));
     }
     if (l == 0 && F->lev0_sparse) {
       Timed tm(c, KORE_TIMER_SPARSE);
@@ -1356,7 +1355,7 @@ template <class T> static int32_t factor_run(kore_sys* s, Factor<T>* F) {
   }
   {
     Timed tm(c, KORE_TIMER_INV);
-    HIP_TRY(launch_gj_inverse<T>(F->root_inv, 1, F->root_n, F->root_n, st));
+    HIP_TRY(launch_gj_inverse<T>(F->root_inv, 1, F->root_n, st));
   }
   if (F->tail) {
     {

@@ -489,6 +489,80 @@ hipError_t launch_skinny1(const SkinnyDesc<T>& d, int nrhs, hipStream_t s) {
 }
 template hipError_t launch_skinny1<double>(const SkinnyDesc<double>&, int, hipStream_t);
 
+// Three and more right-hand sides: Y = beta Y + sum_p alpha_p A_p X_p on the matrix
+// cores, 16 rows by 16 columns per workgroup (unused columns repeat the last).
+// The k of a product stand in groups of four, which the NW waves take in turn:
+// lane (lq, l16) loads A[r0 + l16][4 g + lq] (16 lanes read 256 consecutive bytes)
+// and X[4 g + lq][l16] straight into registers, SKM_NB groups requested before the
+// first is used; the waves' sums are added through LDS.  Bound by the memory
+// round trips on few blocks and by reading A (with X from L2) on many.
+// Measured against the vector kernel, us per launch of complex128 products of
+// 200 rows: 16 columns, 150 blocks 102 -> 35 (one product each) and 162 -> 67
+// (two), one block 19 -> 7 and 30 -> 11; 8 columns 47 -> 32 and 78 -> 58, one block
+// 18 -> 10.  Eight waves instead of four: no faster on one block, 40 and 69 us on 150.
+constexpr int SKM_NB = 8;
+
+template <class T, int NW>
+__global__ __launch_bounds__(64 * NW) void skinny_mm_kernel(const SkinnyDesc<T>* __restrict__ descs, int nrhs) {
+  using A4 = typename acc4<T>::type;
+  const SkinnyDesc<T>& d = descs[blockIdx.y];   // read in place (uniform loads, no private copy)
+  const int r0 = blockIdx.x * SK_ROWS;
+  if (r0 >= d.m) return;
+  __shared__ cx<T> sP[NW][16][SK_ROWS];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int l16 = lane & 15, lq = lane >> 4;
+  const int rc = min(r0 + l16, d.m - 1);        // rows past the block repeat its last one (not stored)
+  const int xc = min(l16, nrhs - 1);
+  A4 cre = {0, 0, 0, 0}, cim = {0, 0, 0, 0};
+#pragma unroll 1
+  for (int p = 0; p < 3; ++p) {
+    const int K = d.A[p] != nullptr ? d.k[p] : 0;
+    const int64_t lda = d.lda[p];
+    const T al = d.alpha[p];
+    const unsigned oa = (unsigned)lq * (unsigned)lda + (unsigned)rc;
+    const cx<T>* X = d.X[p] + (int64_t)xc * d.ldx[p] + lq;
+    for (int k0 = 4 * wave; k0 < K; k0 += 4 * NW * SKM_NB) {
+      const cx<T>* A = d.A[p] + (int64_t)k0 * lda;
+      cx<T> a[SKM_NB], x[SKM_NB];
+      if (k0 + 4 * NW * (SKM_NB - 1) + 4 <= K) {
+#pragma unroll
+        for (int t = 0; t < SKM_NB; ++t) {
+          a[t] = gld(A + (int64_t)(4 * NW * t) * lda + oa);
+          x[t] = gld(X + k0 + 4 * NW * t);
+        }
+      } else {                                  // the last groups: missing k count as zero on both sides
+#pragma unroll
+        for (int t = 0; t < SKM_NB; ++t) {
+          const int back = k0 + 4 * NW * t + lq - (K - 1);   // this lane's k past the last one
+          const int kt = 4 * NW * t - max(back, 0);
+          a[t] = gld(A + (int64_t)kt * lda + oa);
+          x[t] = gld(X + k0 + kt);
+          if (back > 0) a[t] = x[t] = czero<T>();
+        }
+      }
+#pragma unroll
+      for (int t = 0; t < SKM_NB; ++t) cmma<T>(cre, cim, a[t], cx<T>{al * x[t].re, al * x[t].im});
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i) sP[wave][mfma_mrow<T>(lq, i)][l16] = cx<T>{cre[i], cim[i]};
+  __syncthreads();
+  const int row = r0 + l16, c = threadIdx.x >> 4;
+  if (c < nrhs && row < d.m) {
+    cx<T> v = sP[0][c][l16];
+#pragma unroll
+    for (int q = 1; q < NW; ++q) v = cadd(v, sP[q][c][l16]);
+    cx<T>* y = d.Y + (int64_t)c * d.ldy + row;
+    if (d.beta != T(0)) {
+      const cx<T> old = gld(y);
+      v.re += d.beta * old.re;
+      v.im += d.beta * old.im;
+    }
+    gst(y, v);
+  }
+}
+
 template <class T>
 hipError_t launch_skinny(const SkinnyDesc<T>* d_descs, int ndesc, int max_m, int nrhs, hipStream_t s) {
   if (ndesc <= 0 || max_m <= 0) return hipSuccess;
@@ -496,17 +570,18 @@ hipError_t launch_skinny(const SkinnyDesc<T>* d_descs, int ndesc, int max_m, int
   const dim3 grid((unsigned)((max_m + SK_ROWS - 1) / SK_ROWS), (unsigned)ndesc);
   // the preloading form at every size: measured no slower than the streaming
   // loop on the largest sweep levels (thousands of workgroups) and faster on
-  // the deep levels, where a launch holds a handful of blocks
+  // the deep levels, where a launch holds a handful of blocks.  Three or four
+  // columns of blocks of 129 to 256 rows stay on it too (complex64, 200 rows, 150
+  // blocks of two products: 31 us against 36 on the matrix cores; 100 rows 16
+  // against 15, 374 rows, 37 blocks 45 against 31)
   if (nrhs == 1)
     hipLaunchKernelGGL((skinny_kernel<T, 1>), grid, dim3(256), 0, s, d_descs, nrhs);
   else if (nrhs <= 2)
     hipLaunchKernelGGL((skinny_kernel<T, 2>), grid, dim3(256), 0, s, d_descs, nrhs);
-  else if (nrhs <= 4)
+  else if (nrhs <= 4 && max_m > 128 && max_m <= 256)
     hipLaunchKernelGGL((skinny_kernel<T, 4>), grid, dim3(256), 0, s, d_descs, nrhs);
-  else if (nrhs <= 8)
-    hipLaunchKernelGGL((skinny_kernel<T, 8>), grid, dim3(256), 0, s, d_descs, nrhs);
   else
-    hipLaunchKernelGGL((skinny_kernel<T, 16>), grid, dim3(256), 0, s, d_descs, nrhs);
+    hipLaunchKernelGGL((skinny_mm_kernel<T, 4>), grid, dim3(256), 0, s, d_descs, nrhs);
   return hipGetLastError();
 }
 template hipError_t launch_skinny<double>(const SkinnyDesc<double>*, int, int, int, hipStream_t);

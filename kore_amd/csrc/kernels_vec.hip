@@ -563,18 +563,153 @@ __global__ __launch_bounds__(64 * NW) void skinny_mm_kernel(const SkinnyDesc<T>*
   }
 }
 
+// One or two right-hand sides, launches of many workgroups: the operands go
+// straight from memory to registers, as in skinny_mm_kernel, and a complex64 lane
+// takes two rows, so that its loads are 16 bytes and 16 lanes read 256 consecutive
+// ones.  Bound by reading A from HBM.  Measured against the kernel that stages X in
+// LDS, us per launch, 150 blocks of two products: complex64, one column, 374 rows
+// 94 -> 76 (4.5 TB/s), 437 rows 128 -> 102, 500 rows 149 -> 125 (4.9 TB/s); complex128,
+// two columns, 374 rows 142 -> 137 (4.9 TB/s).
+constexpr int SKR_NW = 4, SKR_NB = 8;
+template <class T> constexpr int SKR_ROWS = sizeof(T) == 4 ? 32 : 16;
+template <class T, int RPL> struct row_pack;
+template <> struct row_pack<double, 1> { cx<double> r[1]; };
+template <> struct row_pack<float, 2> { cx<float> r[2]; };
+__device__ __forceinline__ row_pack<double, 1> gld_rows(const cx<double>* p) { return {{gld(p)}}; }
+__device__ __forceinline__ row_pack<float, 2> gld_rows(const cx<float>* p) {
+  typedef float V __attribute__((ext_vector_type(4), aligned(8)));
+  const V v = *(const __attribute__((address_space(1))) V*)p;
+  return {{{v.x, v.y}, {v.z, v.w}}};
+}
+
+template <class T, int NR>
+__global__ __launch_bounds__(64 * SKR_NW) void skinny_row_kernel(const SkinnyDesc<T>* __restrict__ descs, int nrhs) {
+  constexpr int NW = SKR_NW, NB = SKR_NB;
+  constexpr int ROWS = SKR_ROWS<T>, RPL = ROWS / 16;
+  const SkinnyDesc<T>& d = descs[blockIdx.y];   // read in place (uniform loads, no private copy)
+  const int r0 = blockIdx.x * ROWS, m = d.m;
+  if (r0 >= m) return;
+  __shared__ cx<T> sP[NW][NR][ROWS];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int l16 = lane & 15, lq = lane >> 4;
+  const int rc = min(r0 + RPL * l16, m - RPL);  // rows past the block repeat its last ones (not stored); m >= RPL
+  cx<T> acc[NR][RPL];
+#pragma unroll
+  for (int c = 0; c < NR; ++c)
+#pragma unroll
+    for (int q = 0; q < RPL; ++q) acc[c][q] = czero<T>();
+#pragma unroll 1
+  for (int p = 0; p < 3; ++p) {
+    const int K = d.A[p] != nullptr ? d.k[p] : 0;
+    const int64_t lda = d.lda[p], ldx = d.ldx[p];
+    const T al = d.alpha[p];
+    const unsigned oa = (unsigned)lq * (unsigned)lda + (unsigned)rc;
+    cx<T> sum[NR][RPL];
+#pragma unroll
+    for (int c = 0; c < NR; ++c)
+#pragma unroll
+      for (int q = 0; q < RPL; ++q) sum[c][q] = czero<T>();
+    for (int k0 = 4 * wave; k0 < K; k0 += 4 * NW * NB) {
+      const cx<T>* A = d.A[p] + (int64_t)k0 * lda;
+      const cx<T>* X = d.X[p] + k0;
+      row_pack<T, RPL> a[NB];
+      cx<T> x[NB][NR];
+      if (k0 + 4 * NW * (NB - 1) + 4 <= K) {
+#pragma unroll
+        for (int t = 0; t < NB; ++t) {
+          a[t] = gld_rows(A + (int64_t)(4 * NW * t) * lda + oa);
+#pragma unroll
+          for (int c = 0; c < NR; ++c) x[t][c] = gld(X + (c < nrhs ? c : 0) * ldx + 4 * NW * t + lq);
+        }
+      } else {                                  // the last groups: missing k count as zero on both sides
+#pragma unroll
+        for (int t = 0; t < NB; ++t) {
+          const int back = k0 + 4 * NW * t + lq - (K - 1);   // this lane's k past the last one
+          const int kt = 4 * NW * t - max(back, 0);
+          a[t] = gld_rows(A + (int64_t)kt * lda + oa);
+#pragma unroll
+          for (int c = 0; c < NR; ++c) {
+            x[t][c] = gld(X + (c < nrhs ? c : 0) * ldx + kt + lq);
+            if (back > 0) x[t][c] = czero<T>();
+          }
+          if (back > 0)
+#pragma unroll
+            for (int q = 0; q < RPL; ++q) a[t].r[q] = czero<T>();
+        }
+      }
+#pragma unroll
+      for (int t = 0; t < NB; ++t)
+#pragma unroll
+        for (int c = 0; c < NR; ++c)
+#pragma unroll
+          for (int q = 0; q < RPL; ++q) sum[c][q] = cfma(sum[c][q], a[t].r[q], x[t][c]);
+    }
+#pragma unroll
+    for (int c = 0; c < NR; ++c)
+#pragma unroll
+      for (int q = 0; q < RPL; ++q) {
+        acc[c][q].re += al * sum[c][q].re;
+        acc[c][q].im += al * sum[c][q].im;
+      }
+  }
+#pragma unroll
+  for (int c = 0; c < NR; ++c)
+#pragma unroll
+    for (int q = 0; q < RPL; ++q) {
+#pragma unroll
+      for (int off = 16; off <= 32; off *= 2) {
+        acc[c][q].re += __shfl_xor(acc[c][q].re, off, 64);
+        acc[c][q].im += __shfl_xor(acc[c][q].im, off, 64);
+      }
+      if (lq == 0) sP[wave][c][RPL * l16 + q] = acc[c][q];
+    }
+  __syncthreads();
+  const int i = threadIdx.x % ROWS, c = threadIdx.x / ROWS;
+  const int row = r0 + i;
+  // the last row of an odd block is the second one of its lane's pair
+  const int at = RPL == 2 && row == m - 1 && (i & 1) == 0 ? i + 1 : i;
+  if (c < nrhs && c < NR && row < m) {
+    cx<T> v = sP[0][c][at];
+#pragma unroll
+    for (int q = 1; q < NW; ++q) v = cadd(v, sP[q][c][at]);
+    cx<T>* y = d.Y + (int64_t)c * d.ldy + row;
+    if (d.beta != T(0)) {
+      const cx<T> old = gld(y);
+      v.re += d.beta * old.re;
+      v.im += d.beta * old.im;
+    }
+    gst(y, v);
+  }
+}
+
 template <class T>
 hipError_t launch_skinny(const SkinnyDesc<T>* d_descs, int ndesc, int max_m, int nrhs, hipStream_t s) {
   if (ndesc <= 0 || max_m <= 0) return hipSuccess;
   if (nrhs < 1 || nrhs > 16) return hipErrorInvalidValue;
   const dim3 grid((unsigned)((max_m + SK_ROWS - 1) / SK_ROWS), (unsigned)ndesc);
+  // one or two columns from 400 workgroups of skinny_row_kernel (complex64: 37
+  // blocks of 374 rows, 444 workgroups, 27 -> 23 us, 37 of 200 rows, 259, 9 -> 11;
+  // complex128 with two columns 42 -> 40 at 888, with one 39 either way, so that
+  // stays).  Its lanes want two rows and more: a degree's block holds the rows of
+  // one to four fields, so a list whose largest block has 64 has none below 16.
+  const dim3 wgrid((unsigned)((max_m + SKR_ROWS<T> - 1) / SKR_ROWS<T>), (unsigned)ndesc);
+  const bool wide = max_m >= 64 && (int64_t)wgrid.x * wgrid.y >= 400;
   // the preloading form at every size: measured no slower than the streaming
   // loop on the largest sweep levels (thousands of workgroups) and faster on
   // the deep levels, where a launch holds a handful of blocks.  Three or four
   // columns of blocks of 129 to 256 rows stay on it too (complex64, 200 rows, 150
   // blocks of two products: 31 us against 36 on the matrix cores; 100 rows 16
   // against 15, 374 rows, 37 blocks 45 against 31)
-  if (nrhs == 1)
+  if constexpr (sizeof(T) == 4) {
+    if (wide && nrhs == 1) {
+      hipLaunchKernelGGL((skinny_row_kernel<T, 1>), wgrid, dim3(64 * SKR_NW), 0, s, d_descs, nrhs);
+      return hipGetLastError();
+    }
+  }
+  if (wide && nrhs == 2)
+    hipLaunchKernelGGL((skinny_row_kernel<T, 2>), wgrid, dim3(64 * SKR_NW), 0, s, d_descs, nrhs);
+  else if (nrhs == 1)
     hipLaunchKernelGGL((skinny_kernel<T, 1>), grid, dim3(256), 0, s, d_descs, nrhs);
   else if (nrhs <= 2)
     hipLaunchKernelGGL((skinny_kernel<T, 2>), grid, dim3(256), 0, s, d_descs, nrhs);

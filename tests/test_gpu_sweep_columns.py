@@ -36,3 +36,28 @@ def test_columns(ctx, N, precision):
         err = np.linalg.norm(x - xr[:, :k], axis=0) / np.linalg.norm(xr[:, :k], axis=0)
         assert err.max() <= 1e-10
     S.close()
+
+
+@pytest.mark.parametrize("N,lmax", [(63, 830), (64, 830), (65, 830), (77, 550)])
+@pytest.mark.parametrize("precision", [0, 1])
+def test_many_blocks(ctx, N, lmax, precision):
+    """Sweeps with one and two columns over launches of few and of many
+    workgroups, odd block sizes: residual of the refined solution, 1e-13 of
+    |A - sigma B| |x| + |b| by rows (the refinement's own stopping size is
+    1e-14 of the solution)."""
+    from kore_amd import assembly, backend
+    from kore_amd.params import Params
+    par = Params(m=1, symm=1, Ek=1e-4, N=N, lmax=lmax)
+    A, B, _ = assembly.assemble(par)
+    S = backend.System(ctx, backend.layout_from_params(par), A, B)
+    sigma = 0.4j
+    M = (A - sigma * B).tocsr()
+    rng = np.random.default_rng(N)
+    b = rng.standard_normal((S.n, 2)) + 1j * rng.standard_normal((S.n, 2))
+    S.factor(sigma, precision)
+    for k in (1, 2):
+        print("case: many blocks", N, lmax, "precision", precision, "columns", k, flush=True)
+        x, _ = S.solve(b[:, :k], ir_tol=1e-14, ir_maxit=20)
+        r = np.abs(b[:, :k] - M @ x) / (abs(M) @ np.abs(x) + np.abs(b[:, :k]))
+        assert r.max() <= 1e-13
+    S.close()

@@ -17,14 +17,14 @@ template <class T> struct GemmDesc {
   T alpha, beta;
 };
 
-// in-place inverse of an n x n column-major block
+// inverse of an n x n column-major block
 template <class T> struct InvDesc {
-  cx<T>* M;
+  cx<T>* M;         // the block; eliminated in place, holds nothing of use afterwards
   int64_t ld;
   int n;
   int* ipiv;        // n ints of device scratch (pivot row of each column)
   int* info;        // 0 or (1-based column of the first zero pivot)
-  cx<T>* scratch;   // n x n block used for the final permutation
+  cx<T>* scratch;   // n x n: scratch of the elimination, then the inverse
 };
 
 // Y = beta*Y + sum_p alpha_p A_p X_p  (p < 3) for skinny X (nrhs <= 16

@@ -611,7 +611,9 @@ template <class T> struct Factor : FactorBase {
       if (g) hipGraphExecDestroy(g);
   }
   DevBuf mem, aux, desc, vecs;
-  std::vector<cx<T>*> D, L, U, G, H;   // G = Dinv L, H = Dinv U of eliminated blocks
+  // D: inverse diagonal blocks.  G = Dinv L, H = Dinv U of eliminated blocks; until
+  // its inversion a diagonal block stands in its G, from where the inverse goes to D
+  std::vector<cx<T>*> D, L, U, G, H;
   std::vector<Level<T>> lev;
   InvDesc<T>* root_inv = nullptr;
   SkinnyDesc<T>* root_solve = nullptr;
@@ -643,7 +645,7 @@ template <class T> struct Factor : FactorBase {
   cx<T>* Bv = nullptr;  // solve vectors, sizmat x 16, degree-major
   cx<T>* Xv = nullptr;
   int nblk = 0;
-  int64_t ndlu = 0;    // elements of the D/L/U region (cleared before the scatter)
+  int64_t nglu = 0;    // elements of the G/L/U region (cleared before the scatter)
 };
 
 struct kore_sys {
@@ -739,7 +741,7 @@ struct FactorPlan {
   bool sp0 = false;
   std::vector<int64_t> offD, offL, offU, offG, offH;
   std::vector<std::vector<int64_t>> offE, offF;
-  int64_t cntD = 0, cntDLU = 0, cnt = 0;
+  int64_t cntG = 0, cntGLU = 0, cnt = 0;
 };
 
 static void factor_plan(const std::vector<int>& bsz, FactorPlan& P, bool allow_sparse0, bool lean) {
@@ -768,10 +770,10 @@ static void factor_plan(const std::vector<int>& bsz, FactorPlan& P, bool allow_s
   P.offG.assign(nb, -1);
   P.offH.assign(nb, -1);
   for (int k = 0; k < nb; ++k) {
-    P.offD[k] = cnt;
-    cnt += nk(k) * nk(k);
+    P.offG[k] = cnt;
+    cnt += nk(k) * nmax;
   }
-  P.cntD = cnt;
+  P.cntG = cnt;
   for (int k = 0; k < nb; ++k) {
     if (P.sp0 && (k & 1)) continue;        // eliminated at level 0: couplings read from the matrix
     if (k > 0) {
@@ -783,10 +785,10 @@ static void factor_plan(const std::vector<int>& bsz, FactorPlan& P, bool allow_s
       cnt += nk(k) * nmax;
     }
   }
-  P.cntDLU = cnt;
+  P.cntGLU = cnt;
   for (int k = 0; k < nb; ++k) {
-    P.offG[k] = cnt;
-    cnt += nk(k) * nmax;
+    P.offD[k] = cnt;
+    cnt += nk(k) * nk(k);
     P.offH[k] = cnt;
     cnt += nk(k) * nmax;
   }
@@ -954,7 +956,7 @@ template <class T> static int32_t factor_build(kore_sys* s, Factor<T>* F) {
     rinv[l].off = vinv.size();
     for (int t = 1; t < T_; t += 2) {
       const int k = id[t];
-      vinv.push_back(InvDesc<T>{F->D[k], nk(k), (int)nk(k), ipiv + (size_t)k * nmax, F->info + k, F->G[k]});
+      vinv.push_back(InvDesc<T>{F->G[k], nk(k), (int)nk(k), ipiv + (size_t)k * nmax, F->info + k, F->D[k]});
       flops += 8.0 * nk(k) * nk(k) * nk(k);
       F->flops_inv += 8.0 * nk(k) * nk(k) * nk(k);
       L.maxn_inv = std::max(L.maxn_inv, (int)nk(k));
@@ -979,7 +981,7 @@ template <class T> static int32_t factor_build(kore_sys* s, Factor<T>* F) {
       for (int t = 0; t < T_; t += 2) {
         const bool hasE = t - 1 >= 0, hasF = t + 1 <= T_ - 1;
         if (hasE || hasF) {
-          vsr.push_back(mksprow(F->D[t], t, (int)nk(t),
+          vsr.push_back(mksprow(F->G[t], t, (int)nk(t),
                                 {SProd{hasE ? F->H[t - 1] : nullptr, 0}, SProd{hasF ? F->G[t + 1] : nullptr, 1}},
                                 T(-1), T(1)));
           L.maxn_sr = std::max(L.maxn_sr, (int)nk(t));
@@ -1039,7 +1041,7 @@ template <class T> static int32_t factor_build(kore_sys* s, Factor<T>* F) {
         const bool hasE = t - 1 >= 0, hasF = t + 1 <= T_ - 1;
         if (hasE || hasF) {
           const int kp = hasE ? id[t - 1] : -1, kn = hasF ? id[t + 1] : -1;
-          vg.push_back(mkgemm(F->D[k], m, m, hasE ? Lp(l, t) : nullptr, hasE ? F->H[kp] : nullptr,
+          vg.push_back(mkgemm(F->G[k], m, m, hasE ? Lp(l, t) : nullptr, hasE ? F->H[kp] : nullptr,
                               hasE ? (int)nk(kp) : 0, m, hasE ? (int)nk(kp) : 0, hasF ? Up(l, t) : nullptr,
                               hasF ? F->G[kn] : nullptr, hasF ? (int)nk(kn) : 0, m, hasF ? (int)nk(kn) : 0, T(-1),
                               T(1)));
@@ -1139,7 +1141,7 @@ template <class T> static int32_t factor_build(kore_sys* s, Factor<T>* F) {
       const bool hasE = t - 1 >= 0, hasF = t + 1 <= T_ - 1;
       if (hasE || hasF) {
         const int kp = hasE ? id[t - 1] : -1, kn = hasF ? id[t + 1] : -1;
-        vg.push_back(mkgemm(F->D[k], m, m, hasE ? base + P.offE[l][t] : nullptr, hasE ? F->U[kp] : nullptr,
+        vg.push_back(mkgemm(F->G[k], m, m, hasE ? base + P.offE[l][t] : nullptr, hasE ? F->U[kp] : nullptr,
                             hasE ? (int)nk(kp) : 0, m, hasE ? (int)nk(kp) : 0, hasF ? base + P.offF[l][t] : nullptr,
                             hasF ? F->L[kn] : nullptr, hasF ? (int)nk(kn) : 0, m, hasF ? (int)nk(kn) : 0, T(-1),
                             T(1)));
@@ -1194,7 +1196,7 @@ template <class T> static int32_t factor_build(kore_sys* s, Factor<T>* F) {
   // root
   const int kr = ids[nlev][0];
   rinv[nlev].off = vinv.size();
-  vinv.push_back(InvDesc<T>{F->D[kr], nk(kr), (int)nk(kr), ipiv + (size_t)kr * nmax, F->info + kr, F->G[kr]});
+  vinv.push_back(InvDesc<T>{F->G[kr], nk(kr), (int)nk(kr), ipiv + (size_t)kr * nmax, F->info + kr, F->D[kr]});
   rinv[nlev].n = 1;
   flops += 8.0 * nk(kr) * nk(kr) * nk(kr);
   F->flops_inv += 8.0 * nk(kr) * nk(kr) * nk(kr);
@@ -1276,10 +1278,10 @@ template <class T> static int32_t factor_build(kore_sys* s, Factor<T>* F) {
   HIP_TRY(hipMemcpyAsync(dsk, vs.data(), bsk, hipMemcpyHostToDevice, c->stream));
   if (bsc) HIP_TRY(hipMemcpyAsync(dsc, vsc.data(), bsc, hipMemcpyHostToDevice, c->stream));
   if (bsr) HIP_TRY(hipMemcpyAsync(dsr, vsr.data(), bsr, hipMemcpyHostToDevice, c->stream));
-  // the level-0 scatter fills D, and L, U only when level 0 runs on dense couplings
+  // the level-0 scatter fills the diagonal blocks (in G), and L, U only when level 0 runs on dense couplings
   std::vector<cx<T>*> hp(3 * (size_t)nb, nullptr);
   for (int k = 0; k < nb; ++k) {
-    hp[k] = F->D[k];
+    hp[k] = F->G[k];
     hp[nb + k] = sp0 ? nullptr : F->L[k];
     hp[2 * nb + k] = sp0 ? nullptr : F->U[k];
   }
@@ -1304,7 +1306,7 @@ template <class T> static int32_t factor_build(kore_sys* s, Factor<T>* F) {
     F->tail2 = dg + rtail2;
     F->tail_solve = dsk + rtails;
   }
-  F->ndlu = sp0 ? P.cntD : P.cntDLU;
+  F->nglu = sp0 ? P.cntG : P.cntGLU;
   return KORE_OK;
 }
 
@@ -1326,7 +1328,7 @@ template <class T> static int32_t factor_run(kore_sys* s, Factor<T>* F) {
   hipStream_t st = c->stream;
   {
     Timed tm(c, KORE_TIMER_OTHER);
-    HIP_TRY(launch_zero<T>(F->mem.template as<cx<T>>(), F->ndlu, st));
+    HIP_TRY(launch_zero<T>(F->mem.template as<cx<T>>(), F->nglu, st));
     HIP_TRY(launch_build_blocks<T>(s->csr, s->sre, s->sim, s->d_scale.as<double>(), s->d_blk.as<int32_t>(),
                                    s->d_boff.as<int64_t>(), F->dD, F->dL, F->dU, st));
   }

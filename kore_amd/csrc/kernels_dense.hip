@@ -233,27 +233,6 @@ __device__ __forceinline__ void gemm_tile_body(const GemmDesc<T>& d, const int t
   }
 }
 
-// Workgroup id -> (item, part of the item), for launches of `per` workgroups per
-// item.  Consecutive workgroups go to the chip's eight dies in turn, each with
-// its own L2: all parts of an item are kept on one die, so that what
-// they share is fetched into one L2 and not into eight.  That needs many items
-// (a few would leave dies idle): 64 and more.  Measured, complex128 products:
-// 298 of 200 rows 583 -> 520 us, 298 of 500 rows 5.22 -> 5.07 ms.
-constexpr int XCD_MIN_ITEMS = 64;
-__device__ __forceinline__ void xcd_item(int id, int per, int nitems, int& item, int& part) {
-  if (nitems >= XCD_MIN_ITEMS) {
-    const int slot = id >> 3;
-    item = (slot / per) * 8 + (id & 7);
-    part = slot % per;
-  } else {
-    item = id / per;
-    part = id % per;
-  }
-}
-static inline unsigned xcd_grid(int items, int per) {
-  return (unsigned)(items >= XCD_MIN_ITEMS ? (items + 7) / 8 * 8 : items) * (unsigned)per;
-}
-
 // Tile edge 32 instead of 64: where it covers much less padding (n = 200: 224
 // rows instead of 256; n = 150: 160 instead of 192), and where the launch holds
 // few tiles, so that four times the workgroups fill the chip.  Measured, us per

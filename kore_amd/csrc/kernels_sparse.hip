@@ -18,6 +18,7 @@
 //          backward), for complex128 or complex64 vectors and up to 16
 //          right-hand sides
 //   offvals   oval[q] = r_i (a_k - sigma b_k) for the off-block entries
+#include <type_traits>
 #include "kore_device.hpp"
 #include "kore_kernels.hpp"
 
@@ -57,43 +58,42 @@ hipError_t launch_offvals(const CsrDev& m, double sre, double sim, const double*
 }
 
 // ---------------------------------------------------------------------------
-// sparse rows x dense: one workgroup per (descriptor, tile of SR_NC<T>
-// columns).  The tile of each X_p (all its rows, SR_NC columns) is staged in
-// LDS once, so every sparse entry reads its X values from LDS: an entry of
-// column c is shared by the ~w rows of the band around c, which would
-// otherwise re-read X[c, :] from the caches w times.  Each thread owns up to
-// two rows of C (blocks of at most 512 rows) and SR_NC columns.
+// sparse rows x dense: one workgroup per (descriptor, tile of NC columns).  The
+// tile of each X_p (all its rows, NC columns) is staged in LDS once, so every
+// sparse entry reads its X values from LDS: an entry of column c is shared by the
+// ~w rows of the band around c, which would otherwise re-read X[c, :] from the
+// caches w times.  A thread owns one row of C and NC columns; MAXM (256 or 512)
+// threads, so that the rows of the largest block are all in flight: two rows one
+// after the other per thread of 256 left two waves per SIMD waiting on the entries'
+// scattered loads (complex128: 500 rows 4400 -> 3500 us, 200 rows 422 -> 335;
+// complex64, 437 rows 2260 -> 1700).  The last, short group of a row's entries is
+// taken entry by entry: as one group of masked ones it measured slower, as did all
+// tiles of a descriptor on one die.
 // ---------------------------------------------------------------------------
-static constexpr int SR_MAXN = 512;   // rows of a degree block (and of an X tile)
 static constexpr int SR_U = 8;        // sparse entries whose loads are in flight together
 
-template <class T, int NC>
-__global__ __launch_bounds__(256) void sprow_kernel(OffCsr o, const SpRowDesc<T>* __restrict__ descs) {
-  __shared__ cx<T> sX[NC * SR_MAXN];      // X tile, column-major: sX[jj * SR_MAXN + c]
+template <class T, int NC, int MAXM>
+__global__ __launch_bounds__(MAXM) void sprow_kernel(OffCsr o, const SpRowDesc<T>* __restrict__ descs) {
+  __shared__ cx<T> sX[NC * MAXM];         // X tile, column-major: sX[jj * MAXM + c]
   const SpRowDesc<T>& d = descs[blockIdx.y];
   const int j0 = blockIdx.x * NC;
   if (j0 >= d.n) return;                  // uniform over the workgroup
   const int nc = d.n - j0 < NC ? d.n - j0 : NC;
-  const int tid = threadIdx.x;
-  cx<double> acc[2][NC];
+  const int r = threadIdx.x, lane = r & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(r >> 6);
+  cx<double> acc[NC];
 #pragma unroll
-  for (int h = 0; h < 2; ++h)
-#pragma unroll
-    for (int c = 0; c < NC; ++c) acc[h][c] = czero<double>();
+  for (int c = 0; c < NC; ++c) acc[c] = czero<double>();
   for (int p = 0; p < 2; ++p) {
     if (d.side[p] < 0) continue;          // uniform
     const int nbk = d.xrows[p];           // rows of X_p (the neighbouring block's unknowns)
     const cx<T>* X = d.X[p] + (int64_t)j0 * d.ldx[p];
     __syncthreads();                      // the previous product's reads are done
-    for (int idx = tid; idx < NC * nbk; idx += 256) {
-      const int jj = idx / nbk, c = idx - jj * nbk;
-      sX[jj * SR_MAXN + c] = jj < nc ? gld(X + (int64_t)jj * d.ldx[p] + c) : czero<T>();
-    }
+    for (int jj = wave; jj < NC; jj += MAXM / 64)
+      for (int c = lane; c < nbk; c += 64)
+        sX[jj * MAXM + c] = jj < nc ? gld(X + (int64_t)jj * d.ldx[p] + c) : czero<T>();
     __syncthreads();
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const int r = tid + 256 * h;
-      if (r >= d.m) continue;
+    if (r < d.m) {
       const int64_t row = d.row0 + r;
       const int s = o.ptr[row], nl = o.nlo[row];
       const int q0 = d.side[p] == 0 ? s : s + nl, q1 = d.side[p] == 0 ? s + nl : o.ptr[row + 1];
@@ -114,33 +114,29 @@ __global__ __launch_bounds__(256) void sprow_kernel(OffCsr o, const SpRowDesc<T>
         for (int u = 0; u < SR_U; ++u) {
           const int c = cc[u] - xc0;
 #pragma unroll
-          for (int jj = 0; jj < NC; ++jj) acc[h][jj] = cfma(acc[h][jj], vv[u], up(sX[jj * SR_MAXN + c]));
+          for (int jj = 0; jj < NC; ++jj) acc[jj] = cfma(acc[jj], vv[u], up(sX[jj * MAXM + c]));
         }
       }
       for (; q < q1; ++q) {
         const cx<double> v = o.val[q];
         const int c = o.col[q] - xc0;
 #pragma unroll
-        for (int jj = 0; jj < NC; ++jj) acc[h][jj] = cfma(acc[h][jj], v, up(sX[jj * SR_MAXN + c]));
+        for (int jj = 0; jj < NC; ++jj) acc[jj] = cfma(acc[jj], v, up(sX[jj * MAXM + c]));
       }
     }
   }
+  if (r >= d.m) return;
 #pragma unroll
-  for (int h = 0; h < 2; ++h) {
-    const int r = tid + 256 * h;
-    if (r >= d.m) continue;
-#pragma unroll
-    for (int jj = 0; jj < NC; ++jj) {
-      if (jj < nc) {
-        cx<T>* y = d.C + (int64_t)(j0 + jj) * d.ldc + r;
-        cx<double> out{(double)d.alpha * acc[h][jj].re, (double)d.alpha * acc[h][jj].im};
-        if (d.beta != T(0)) {
-          const cx<double> old = up(gld(y));
-          out.re += (double)d.beta * old.re;
-          out.im += (double)d.beta * old.im;
-        }
-        gst(y, cx<T>{(T)out.re, (T)out.im});
+  for (int jj = 0; jj < NC; ++jj) {
+    if (jj < nc) {
+      cx<T>* y = d.C + (int64_t)(j0 + jj) * d.ldc + r;
+      cx<double> out{(double)d.alpha * acc[jj].re, (double)d.alpha * acc[jj].im};
+      if (d.beta != T(0)) {
+        const cx<double> old = up(gld(y));
+        out.re += (double)d.beta * old.re;
+        out.im += (double)d.beta * old.im;
       }
+      gst(y, cx<T>{(T)out.re, (T)out.im});
     }
   }
 }
@@ -149,34 +145,50 @@ __global__ __launch_bounds__(256) void sprow_kernel(OffCsr o, const SpRowDesc<T>
 // complex128, so 128 KiB of gfx950's 160 KiB at 16; half that for complex64);
 // chosen per block-size class by the library's tuner.
 template <class T>
-hipError_t launch_sprow(const OffCsr& o, const SpRowDesc<T>* d_descs, int ndesc, int max_m, int max_n, int nc,
-                        hipStream_t s) {
+hipError_t launch_sprow(const OffCsr& o, const SpRowDesc<T>* d_descs, int ndesc, int max_m, int max_x, int max_n,
+                        int nc, hipStream_t s) {
   if (ndesc <= 0 || max_m <= 0 || max_n <= 0) return hipSuccess;
-  if (max_m > SR_MAXN) return hipErrorInvalidValue;
+  if (max_m > 512) return hipErrorInvalidValue;
   const dim3 grid((unsigned)((max_n + nc - 1) / nc), (unsigned)ndesc);
+  auto launch = [&](auto tile) {
+    constexpr int NC = decltype(tile)::value;
+    if (max_m <= 256 && max_x <= 256)
+      hipLaunchKernelGGL((sprow_kernel<T, NC, 256>), grid, dim3(256), 0, s, o, d_descs);
+    else
+      hipLaunchKernelGGL((sprow_kernel<T, NC, 512>), grid, dim3(512), 0, s, o, d_descs);
+  };
   if (nc == 4)
-    hipLaunchKernelGGL((sprow_kernel<T, 4>), grid, dim3(256), 0, s, o, d_descs);
+    launch(std::integral_constant<int, 4>{});
   else if (nc == 8)
-    hipLaunchKernelGGL((sprow_kernel<T, 8>), grid, dim3(256), 0, s, o, d_descs);
+    launch(std::integral_constant<int, 8>{});
   else if (nc == 16)
-    hipLaunchKernelGGL((sprow_kernel<T, 16>), grid, dim3(256), 0, s, o, d_descs);
+    launch(std::integral_constant<int, 16>{});
   else
     return hipErrorInvalidValue;
   return hipGetLastError();
 }
-template hipError_t launch_sprow<double>(const OffCsr&, const SpRowDesc<double>*, int, int, int, int, hipStream_t);
-template hipError_t launch_sprow<float>(const OffCsr&, const SpRowDesc<float>*, int, int, int, int, hipStream_t);
+template hipError_t launch_sprow<double>(const OffCsr&, const SpRowDesc<double>*, int, int, int, int, int,
+                                         hipStream_t);
+template hipError_t launch_sprow<float>(const OffCsr&, const SpRowDesc<float>*, int, int, int, int, int,
+                                        hipStream_t);
 
 // ---------------------------------------------------------------------------
 // dense x sparse columns: one wave per output column, lanes over the rows;
 // the column's entry list is uniform over the wave (scalar loads) and each
-// entry is one coalesced column segment of X
+// entry is one coalesced column segment of X.  Bound by reading X, of which
+// neighbouring columns use the same parts: all columns of a descriptor stay on one
+// die's L2 (298 blocks of 500 rows, complex128: 2310 -> 2050 us), and a column's last,
+// short group of entries waits for memory once and not per entry (-> 1700; complex64
+// 437 rows 1340 -> 830).  Two chunks of rows at once: no faster.
 // ---------------------------------------------------------------------------
 template <class T>
 __global__ __launch_bounds__(256) void spcol_kernel(OffCsc cc, const cx<double>* __restrict__ oval,
-                                                    const SpColDesc<T>* __restrict__ descs) {
-  const SpColDesc<T>& d = descs[blockIdx.y];
-  const int c = blockIdx.x * 4 + (threadIdx.x >> 6);
+                                                    const SpColDesc<T>* __restrict__ descs, int ndesc, int per) {
+  int di, tile;
+  xcd_item(blockIdx.x, per, ndesc, di, tile);
+  if (di >= ndesc) return;
+  const SpColDesc<T>& d = descs[di];
+  const int c = tile * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
   if (c >= d.n) return;
   const int k0 = cc.ptr[d.cbase + c], k1 = cc.ptr[d.cbase + c + 1];
@@ -184,22 +196,20 @@ __global__ __launch_bounds__(256) void spcol_kernel(OffCsc cc, const cx<double>*
     const int r = r0 + lane;
     cx<double> acc = czero<double>();
     if (r < d.m) {
-      // entries in groups of SR_U, loads first (as in sprow_kernel)
-      int k = k0;
-      for (; k + SR_U <= k1; k += SR_U) {
+      // entries in groups of SR_U, loads first (as in sprow_kernel); the last
+      // group's missing entries repeat the last one's loads and are not added
+      for (int k = k0; k < k1; k += SR_U) {
         cx<double> vv[SR_U];
         cx<T> xx[SR_U];
 #pragma unroll
         for (int u = 0; u < SR_U; ++u) {
-          vv[u] = oval[cc.q[k + u]];
-          xx[u] = gld(d.X + (int64_t)cc.row[k + u] * d.ldx + r);
+          const int ku = min(k + u, k1 - 1);
+          vv[u] = oval[cc.q[ku]];
+          xx[u] = gld(d.X + (int64_t)cc.row[ku] * d.ldx + r);
         }
 #pragma unroll
-        for (int u = 0; u < SR_U; ++u) acc = cfma(acc, up(xx[u]), vv[u]);
-      }
-      for (; k < k1; ++k) {
-        const cx<double> v = oval[cc.q[k]];
-        acc = cfma(acc, up(gld(d.X + (int64_t)cc.row[k] * d.ldx + r)), v);
+        for (int u = 0; u < SR_U; ++u)
+          if (k + u < k1) acc = cfma(acc, up(xx[u]), vv[u]);      // uniform
       }
       cx<T>* y = d.C + (int64_t)c * d.ldc + r;
       cx<double> out{(double)d.alpha * acc.re, (double)d.alpha * acc.im};
@@ -217,8 +227,8 @@ template <class T>
 hipError_t launch_spcol(const OffCsc& cc, const cx<double>* oval, const SpColDesc<T>* d_descs, int ndesc, int max_n,
                         hipStream_t s) {
   if (ndesc <= 0 || max_n <= 0) return hipSuccess;
-  const dim3 grid((unsigned)((max_n + 3) / 4), (unsigned)ndesc);
-  hipLaunchKernelGGL(spcol_kernel<T>, grid, dim3(256), 0, s, cc, oval, d_descs);
+  const int per = (max_n + 3) / 4;
+  hipLaunchKernelGGL(spcol_kernel<T>, dim3(xcd_grid(ndesc, per)), dim3(256), 0, s, cc, oval, d_descs, ndesc, per);
   return hipGetLastError();
 }
 template hipError_t launch_spcol<double>(const OffCsc&, const cx<double>*, const SpColDesc<double>*, int, int,

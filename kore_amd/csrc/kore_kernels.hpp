@@ -121,10 +121,10 @@ template <class T> struct SpColDesc {
 };
 hipError_t launch_offvals(const CsrDev& m, double sre, double sim, const double* scale, const int32_t* split,
                           const OffCsr& o, hipStream_t s);
-// nc: columns per workgroup tile (4, 8; 16 for complex64)
+// max_m, max_x: most rows of C and of any X_p; nc: columns per workgroup tile (4, 8, 16)
 template <class T>
-hipError_t launch_sprow(const OffCsr& o, const SpRowDesc<T>* d_descs, int ndesc, int max_m, int max_n, int nc,
-                        hipStream_t s);
+hipError_t launch_sprow(const OffCsr& o, const SpRowDesc<T>* d_descs, int ndesc, int max_m, int max_x, int max_n,
+                        int nc, hipStream_t s);
 template <class T>
 hipError_t launch_spcol(const OffCsc& cc, const cx<double>* oval, const SpColDesc<T>* d_descs, int ndesc, int max_n,
                         hipStream_t s);

@@ -1342,7 +1342,7 @@ template <class T> static int32_t factor_run(kore_sys* s, Factor<T>* F) {
       Timed tm(c, KORE_TIMER_SPARSE);
       HIP_TRY(launch_spcol<T>(s->offc, s->off.val, L.sc, L.nsc, L.maxn_sc, st));
       if (F->tune_ev[0]) HIP_TRY(hipEventRecord(F->tune_ev[0], st));
-      HIP_TRY(launch_sprow<T>(s->off, L.sr, L.nsr, L.maxm_sr, L.maxn_sr, F->sprow_nc, st));
+      HIP_TRY(launch_sprow<T>(s->off, L.sr, L.nsr, L.maxm_sr, s->nmax, L.maxn_sr, F->sprow_nc, st));
       if (F->tune_ev[1]) HIP_TRY(hipEventRecord(F->tune_ev[1], st));
       continue;
     }

@@ -237,11 +237,12 @@ template <int NR> struct SkPreK { static constexpr int value = NR <= 2 ? 512 : S
 // memory round trip instead of one per product.  Products are accumulated in
 // the same order, with the same alpha-scaled X values, as the per-product form.
 // NP: products held in registers (3; 1 for launches whose descriptors hold one).
-template <class T, int NR, int NP>
+// KS: k-slices of the workgroup (16 KS threads); 16 KS k entries fit.
+template <class T, int NR, int NP, int KS = SK_KS>
 __device__ __forceinline__ void skinny_fused_pre(const SkinnyDesc<T>& d, int nrhs, int row, int ks, cx<T> (&acc)[NR]) {
-  constexpr int NA = SK_PRE_K / SK_KS;               // A entries per thread and product
-  constexpr int NXL = (SK_PRE_K * NR + 255) / 256;   // X entries per thread and product
-  __shared__ cx<T> sXf[NP][SK_PRE_K][NR];
+  constexpr int NA = 16, KMAX = NA * KS, NT = SK_ROWS * KS;   // A entries per thread and product
+  constexpr int NXL = (KMAX * NR + NT - 1) / NT;     // X entries per thread and product
+  __shared__ cx<T> sXf[NP][KMAX][NR];
   cx<T> xr[NP][NXL];
   cx<T> a[NP][NA];
 #pragma unroll
@@ -251,10 +252,10 @@ __device__ __forceinline__ void skinny_fused_pre(const SkinnyDesc<T>& d, int nrh
     const int64_t ldx = d.ldx[p];
 #pragma unroll
     for (int t = 0; t < NXL; ++t) {
-      const int idx = threadIdx.x + 256 * t;
+      const int idx = threadIdx.x + NT * t;
       const int kk = idx / NR, c = idx - kk * NR;
       xr[p][t] = czero<T>();
-      if (idx < SK_PRE_K * NR && kk < K && c < nrhs) xr[p][t] = gld(X + (int64_t)c * ldx + kk);
+      if (idx < KMAX * NR && kk < K && c < nrhs) xr[p][t] = gld(X + (int64_t)c * ldx + kk);
     }
   }
 #pragma unroll
@@ -264,7 +265,7 @@ __device__ __forceinline__ void skinny_fused_pre(const SkinnyDesc<T>& d, int nrh
     const int64_t lda = d.lda[p];
 #pragma unroll
     for (int t = 0; t < NA; ++t) {
-      const int kk = ks + SK_KS * t;
+      const int kk = ks + KS * t;
       a[p][t] = czero<T>();
       if (row < d.m && kk < K) a[p][t] = gld(Ac + (int64_t)kk * lda);
     }
@@ -274,8 +275,8 @@ __device__ __forceinline__ void skinny_fused_pre(const SkinnyDesc<T>& d, int nrh
     const T al = d.alpha[p];
 #pragma unroll
     for (int t = 0; t < NXL; ++t) {
-      const int idx = threadIdx.x + 256 * t;
-      if (idx < SK_PRE_K * NR) {
+      const int idx = threadIdx.x + NT * t;
+      if (idx < KMAX * NR) {
         const int kk = idx / NR, c = idx - kk * NR;
         sXf[p][kk][c] = cx<T>{xr[p][t].re * al, xr[p][t].im * al};
       }
@@ -287,7 +288,7 @@ __device__ __forceinline__ void skinny_fused_pre(const SkinnyDesc<T>& d, int nrh
     if (d.A[p] == nullptr || d.k[p] <= 0) continue;   // uniform
 #pragma unroll
     for (int t = 0; t < NA; ++t) {
-      const int kk = ks + SK_KS * t;                  // entries past K are zero on both sides
+      const int kk = ks + KS * t;                  // entries past K are zero on both sides
 #pragma unroll
       for (int c = 0; c < NR; ++c) acc[c] = cfma(acc[c], a[p][t], sXf[p][kk][c]);
     }
@@ -441,6 +442,47 @@ __device__ __forceinline__ void skinny_tile(const SkinnyDesc<T>& d, int nrhs) {
 template <class T, int NR>
 __global__ __launch_bounds__(256) void skinny_kernel(const SkinnyDesc<T>* __restrict__ descs, int nrhs) {
   skinny_tile<T, NR, true>(descs[blockIdx.y], nrhs);   // descriptor read in place (uniform loads, no private copy)
+}
+
+// Launches of few workgroups, one or two right-hand sides, K up to 512: as
+// skinny_fused_pre, with 32 k-slices instead of 16, so that all products of blocks of
+// 257 to 512 rows fit the registers and cost one memory round trip.
+constexpr int SKD_KS = 32;
+template <class T, int NR>
+__global__ __launch_bounds__(SK_ROWS * SKD_KS) void skinny_deep_kernel(const SkinnyDesc<T>* __restrict__ descs, int nrhs) {
+  const SkinnyDesc<T>& d = descs[blockIdx.y];
+  const int r0 = blockIdx.x * SK_ROWS;
+  if (r0 >= d.m) return;
+  constexpr int NW = SK_ROWS * SKD_KS / 64;
+  __shared__ cx<T> sP[NW][NR][SK_ROWS];
+  const int rl = threadIdx.x & (SK_ROWS - 1), row = r0 + rl, wave = threadIdx.x >> 6;
+  cx<T> acc[NR];
+#pragma unroll
+  for (int c = 0; c < NR; ++c) acc[c] = czero<T>();
+  skinny_fused_pre<T, NR, 3, SKD_KS>(d, nrhs, row, threadIdx.x / SK_ROWS, acc);
+#pragma unroll
+  for (int c = 0; c < NR; ++c) {
+#pragma unroll
+    for (int off = 16; off <= 32; off *= 2) {
+      acc[c].re += __shfl_xor(acc[c].re, off, 64);
+      acc[c].im += __shfl_xor(acc[c].im, off, 64);
+    }
+    if ((threadIdx.x & 63) < SK_ROWS) sP[wave][c][rl] = acc[c];
+  }
+  __syncthreads();
+  const int c = threadIdx.x / SK_ROWS;
+  if (c < nrhs && c < NR && row < d.m) {
+    cx<T> v = sP[0][c][rl];
+#pragma unroll
+    for (int q = 1; q < NW; ++q) v = cadd(v, sP[q][c][rl]);
+    cx<T>* y = d.Y + (int64_t)c * d.ldy + row;
+    if (d.beta != T(0)) {
+      const cx<T> old = gld(y);
+      v.re += d.beta * old.re;
+      v.im += d.beta * old.im;
+    }
+    gst(y, v);
+  }
 }
 
 // one right-hand side and at most NP products per descriptor, blocks up to
@@ -695,6 +737,17 @@ hipError_t launch_skinny(const SkinnyDesc<T>* d_descs, int ndesc, int max_m, int
   // one to four fields, so a list whose largest block has 64 has none below 16.
   const dim3 wgrid((unsigned)((max_m + SKR_ROWS<T> - 1) / SKR_ROWS<T>), (unsigned)ndesc);
   const bool wide = max_m >= 64 && (int64_t)wgrid.x * wgrid.y >= 400;
+  // blocks of 257 to 512 rows in at most one workgroup per CU: one memory round trip
+  // whatever the number of products (complex128, two products and columns, 374
+  // rows: one block 11.4 -> 9.3 us, 8 blocks, 192 workgroups, 15.1 -> 13.1; at 14
+  // blocks, 336 workgroups, 20.9 -> 23.6)
+  if (nrhs <= 2 && max_m > 256 && max_m <= 512 && (int64_t)grid.x * grid.y <= 256) {
+    if (nrhs == 1)
+      hipLaunchKernelGGL((skinny_deep_kernel<T, 1>), grid, dim3(SK_ROWS * SKD_KS), 0, s, d_descs, nrhs);
+    else
+      hipLaunchKernelGGL((skinny_deep_kernel<T, 2>), grid, dim3(SK_ROWS * SKD_KS), 0, s, d_descs, nrhs);
+    return hipGetLastError();
+  }
   // the preloading form at every size: measured no slower than the streaming
   // loop on the largest sweep levels (thousands of workgroups) and faster on
   // the deep levels, where a launch holds a handful of blocks.  Three or four

@@ -657,7 +657,12 @@ struct kore_sys {
   std::vector<int64_t> boff;
   std::vector<int64_t> perm;
   std::vector<int32_t> h_ip, h_blk;
-  std::vector<int32_t> h_amap;     // union-pattern position of each entry of the A given at creation (-1: dropped)
+  // union-pattern position of each entry of the A given at creation (-1:
+  // dropped), the positions that no entry of A has, and whether some has several
+  std::unique_ptr<int32_t[]> h_amap;
+  int64_t n_amap = 0;
+  std::vector<int32_t> h_aless;
+  bool a_repeats = false;
   int64_t nnz = 0;                 // entries of the union pattern (device arrays only)
   int64_t off_nnz[2] = {0, 0};     // entries outside the diagonal block, rows of even / odd blocks
   int64_t off_rows[2] = {0, 0};    // rows of even / odd blocks
@@ -1994,22 +1999,19 @@ static int32_t sys_prepare(const kore_layout* lay, int64_t sizmat, const int32_t
   std::vector<int64_t> inv(n);
   for (int64_t i = 0; i < n; ++i) inv[s->perm[i]] = i;
   // validate CSR
-  auto check_csr = [&](const int32_t* ip, const int32_t* ix, const char* nm) -> int32_t {
+  auto check_csr = [&](const int32_t* ip, const char* nm) -> int32_t {
     if (ip[0] != 0) return fail(KORE_ERR_ARG, "%s: indptr[0] != 0", nm);
     for (int64_t r = 0; r < n; ++r) {
       if (ip[r + 1] < ip[r]) return fail(KORE_ERR_ARG, "%s: indptr not monotone at row %lld", nm, (long long)r);
     }
-    const int64_t nnz = ip[n];
-    for (int64_t k = 0; k < nnz; ++k)
-      if (ix[k] < 0 || ix[k] >= n) return fail(KORE_ERR_ARG, "%s: column index out of range", nm);
-    return KORE_OK;
+    return KORE_OK;                       // column indices are checked by the threads that read them
   };
   trace.mark("sys_create layout");
-  TRY(check_csr(a_indptr, a_indices, "A"));
+  TRY(check_csr(a_indptr, "A"));
   s->has_b = b_indptr != nullptr;
   if (s->has_b) {
     if (!b_indices || !b_data) return fail(KORE_ERR_ARG, "B arrays incomplete");
-    TRY(check_csr(b_indptr, b_indices, "B"));
+    TRY(check_csr(b_indptr, "B"));
   }
   // union pattern in degree-major order, built by row ranges on host threads
   // (each range into its own arrays, then concatenated in row order)
@@ -2018,7 +2020,8 @@ static int32_t sys_prepare(const kore_layout* lay, int64_t sizmat, const int32_t
     int32_t src;   // k >= 0: A entry k; k < 0: B entry -(k + 1)
   };
   const int64_t nnz_a = a_indptr[n];
-  s->h_amap.assign((size_t)nnz_a, -1);
+  s->h_amap.reset(new int32_t[(size_t)std::max<int64_t>(nnz_a, 1)]);   // set by the threads that read A
+  s->n_amap = nnz_a;
   const int nth = (int)std::max<int64_t>(1, std::min<int64_t>((int64_t)host_threads(), std::max<int64_t>(1, n / 4096)));
   // per-range upper bounds (entries of A plus B on the range's rows) place
   // each range's output in the pinned arena before anything is built
@@ -2061,6 +2064,8 @@ static int32_t sys_prepare(const kore_layout* lay, int64_t sizmat, const int32_t
   std::vector<int32_t>& rowcntb = P->rowcntb;
   rowcntb.assign(n, 0);
   std::vector<int64_t> bad_row(nth, -1);
+  std::vector<char> bad_a(nth, 0), bad_b(nth, 0), rept(nth, 0);
+  std::vector<std::vector<int32_t>> taless(nth);  // positions without an entry of A (range-local)
   std::vector<int> bad_kb(nth, 0), bad_kc(nth, 0);
   // A row (or B row) in Kore order maps to degree order as a few increasing
   // runs (one per section and degree), disjoint in their columns: ordering
@@ -2111,9 +2116,18 @@ static int32_t sys_prepare(const kore_layout* lay, int64_t sizmat, const int32_t
       const int64_t r = s->perm[i];
       ra.clear();
       rb.clear();
-      for (int32_t k = a_indptr[r]; k < a_indptr[r + 1]; ++k) ra.push_back({(int32_t)inv[a_indices[k]], k});
+      for (int32_t k = a_indptr[r]; k < a_indptr[r + 1]; ++k) {
+        const int32_t col = a_indices[k];
+        s->h_amap[k] = -1;
+        if (col < 0 || col >= n) bad_a[t] = 1;
+        else ra.push_back({(int32_t)inv[col], k});
+      }
       if (s->has_b)
-        for (int32_t k = b_indptr[r]; k < b_indptr[r + 1]; ++k) rb.push_back({(int32_t)inv[b_indices[k]], -(k + 1)});
+        for (int32_t k = b_indptr[r]; k < b_indptr[r + 1]; ++k) {
+          const int32_t col = b_indices[k];
+          if (col < 0 || col >= n) bad_b[t] = 1;
+          else rb.push_back({(int32_t)inv[col], -(k + 1)});
+        }
       // each part sorted by its runs, then the two merged (A before B on equal
       // columns); the buffers are reused from row to row
       sort_runs(ra, sa, runs);
@@ -2155,8 +2169,14 @@ static int32_t sys_prepare(const kore_layout* lay, int64_t sizmat, const int32_t
         // explicit zeros inside the three block diagonals stay in the pattern
         // (kore_sys_update_a may give them values); outside it they are dropped
         if (a == zd(0, 0) && b == zd(0, 0) && !inband) continue;
+        int na = 0;
         for (size_t qq = q0; qq < q; ++qq)
-          if (row[qq].src >= 0) s->h_amap[row[qq].src] = (int32_t)cntt;   // range-local position, fixed below
+          if (row[qq].src >= 0) {
+            s->h_amap[row[qq].src] = (int32_t)cntt;   // range-local position, fixed below
+            ++na;
+          }
+        if (na == 0) taless[t].push_back((int32_t)cntt);
+        if (na > 1) rept[t] = 1;
         if (!inband && bad_row[t] < 0) {
           bad_row[t] = i;
           bad_kb[t] = kb;
@@ -2193,10 +2213,18 @@ static int32_t sys_prepare(const kore_layout* lay, int64_t sizmat, const int32_t
     for (auto& th : pool) th.join();
   }
   trace.mark("sys_create union pattern");
+  for (int t = 0; t < nth; ++t)
+    if (bad_a[t]) return fail(KORE_ERR_ARG, "A: column index out of range");
+  for (int t = 0; t < nth; ++t)
+    if (bad_b[t]) return fail(KORE_ERR_ARG, "B: column index out of range");
   // positions of the A entries: range-local -> global
   {
     std::vector<int64_t> rbase(nth + 1, 0);
     for (int t = 0; t < nth; ++t) rbase[t + 1] = rbase[t] + (int64_t)tcnt[t];
+    for (int t = 0; t < nth; ++t) {
+      for (int32_t q : taless[t]) s->h_aless.push_back((int32_t)(q + rbase[t]));
+      s->a_repeats = s->a_repeats || rept[t];
+    }
     auto fix = [&](int t) {
       const int64_t r0 = n * t / nth, r1 = n * (t + 1) / nth;
       for (int64_t i = r0; i < r1; ++i) {
@@ -2476,18 +2504,37 @@ int32_t kore_sys_update_a(kore_sys* s, const double* a_data) {
   char* arena = nullptr;
   TRY(ctx_pinned(c, (size_t)std::max<int64_t>(s->nnz, 1) * sizeof(zd), &arena));
   zd* va = reinterpret_cast<zd*>(arena);
-  std::fill(va, va + s->nnz, zd(0, 0));
-  for (size_t k = 0; k < s->h_amap.size(); ++k) {
-    const zd v(a_data[2 * k], a_data[2 * k + 1]);
-    const int32_t pos = s->h_amap[k];
-    if (pos < 0) {
-      if (v != zd(0, 0))
-        return fail(KORE_ERR_UNSUPPORTED, "A entry %zu was a zero outside the block-tridiagonal pattern at "
-                    "creation and cannot take a value now", k);
-      continue;
+  // entries of A go to positions of their own (unless the pattern repeats one),
+  // so that threads can place them in any order
+  const int64_t na = s->n_amap;
+  const int nt = s->a_repeats ? 1 : (int)std::max<int64_t>(1, std::min<int64_t>(std::min(8, host_threads()), na >> 15));
+  if (s->a_repeats) std::fill(va, va + s->nnz, zd(0, 0));
+  else
+    for (int32_t q : s->h_aless) va[q] = zd(0, 0);
+  std::vector<int64_t> bad(nt, -1);       // first entry of each range that has no position and a value
+  auto place = [&](int t) {
+    for (int64_t k = na * t / nt; k < na * (t + 1) / nt; ++k) {
+      const zd v(a_data[2 * k], a_data[2 * k + 1]);
+      const int32_t pos = s->h_amap[k];
+      if (pos < 0) {
+        if (v != zd(0, 0) && bad[t] < 0) bad[t] = k;
+      } else if (s->a_repeats) {
+        va[pos] += v;
+      } else {
+        va[pos] = zd(0, 0) + v;           // as a sum from zero gives it (-0 becomes 0)
+      }
     }
-    va[pos] += v;
+  };
+  {
+    std::vector<std::thread> pool;
+    for (int t = 1; t < nt; ++t) pool.emplace_back(place, t);
+    place(0);
+    for (auto& th : pool) th.join();
   }
+  for (int t = 0; t < nt; ++t)
+    if (bad[t] >= 0)
+      return fail(KORE_ERR_UNSUPPORTED, "A entry %lld was a zero outside the block-tridiagonal pattern at "
+                  "creation and cannot take a value now", (long long)bad[t]);
   if (s->nnz > 0)
     HIP_TRY(hipMemcpyAsync(s->d_va.p, va, (size_t)s->nnz * sizeof(zd), hipMemcpyHostToDevice, c->stream));
   HIP_TRY(hipStreamSynchronize(c->stream));

@@ -278,8 +278,8 @@ template <class T> __device__ __forceinline__ T tiny_pivot() { return sizeof(T) 
 // then gj_perm_kernel: A^{-1}[k, l] = M[r_k, r^{-1}(l)] into the scratch block,
 // which is where the inverse is wanted.  Blocks of one panel (up to 32 rows) are complete
 // after gj_panel_kernel, which stores them in their final order: one launch
-// (24 rows, complex128: 55 -> 20 us; a kernel that ran the whole elimination of
-// a block in one workgroup, used below 96 rows, is gone: 74 rows 193 -> 94 us).
+// (24 rows, complex128: 55 -> 19 us; a kernel that ran the whole elimination of
+// a block in one workgroup, used below 96 rows, is gone: 74 rows 193 -> 82 us).
 // Scratch layout (per block of more than 32 rows, n x n complex): R
 // (32 x n, R[k, j] at R[j 32 + k]), then n ints of row roles (-1 unused,
 // c >= 0: the pivot row of column c).  The multi-panel composition: with T
@@ -372,6 +372,134 @@ template <class T, int NMAX> constexpr int GJ_TPR = sizeof(T) == 8 && NMAX > 256
 // columns of a pivot row that a panel keeps in flight: all of an outer panel's
 constexpr int gj_gather_cols(int nmax) { return nmax <= 256 ? nmax : 128; }
 
+template <class T> __device__ __forceinline__ cx<T> cmul_fma(cx<T> a, cx<T> b) {
+  return cx<T>{fma(a.re, b.re, -(a.im * b.im)), fma(a.re, b.im, a.im * b.re)};
+}
+
+// What the column steps of a workgroup share.
+template <class T, int SW> struct GjLds {
+  cx<T> row[2][SW];                       // the pivot row
+  cx<T> inv[SW];                          // minus the inverse pivots
+  unsigned key[4];                        // best key of a step; steps take the four in turn
+  int piv[GJM_WP];                        // pivot row of each of the panel's columns
+  int sing;
+};
+
+template <int CTRL, class T> __device__ __forceinline__ cx<T> dpp_cx(cx<T> x) {
+  return cx<T>{dpp_t<CTRL>(x.re), dpp_t<CTRL>(x.im)};
+}
+
+// Gauss-Jordan on kw <= SW columns, TPR threads per row: this thread's v holds
+// columns [CPT h, CPT h + CPT) of row r.  The columns are j0 .. of the block and
+// s0 .. of the panel.  Returns which of them the row pivots, or -1; v then holds the
+// final columns.  ONCE: a step's product is formed first and rounds each entry once
+// (two fused multiply-adds round it twice), for a third more operations.
+template <class T, int SW, int TPR, bool ONCE>
+__device__ __forceinline__ int gj_eliminate(GjLds<T, SW>& sm, cx<T> (&v)[SW / TPR], int& role, int& sing, int j0,
+                                            int s0, int kw, int zero_off) {
+  constexpr int CPT = SW / TPR;
+  const int r = threadIdx.x / TPR, h = threadIdx.x % TPR;
+  // A step's key is one mask and one or: rows in use have both zero.  Every
+  // column has an unused row left, so the best key is never zero.
+  const unsigned rowkey = 0x80000000u | (unsigned)(511 - r);
+  unsigned rk = role == -1 && h == 0 ? rowkey : 0u, mk = role == -1 && h == 0 ? 0x7FFFFE00u : 0u;
+  unsigned mykey = 0;                   // of the row (of all its lanes)
+  // the row's entry x of column s0 + c enters the search for its pivot
+  auto compete = [&](cx<T> x, int c) __attribute__((always_inline)) {
+    mykey = (pivot_bits(cabs1(x)) & mk) | rk;
+    unsigned key = mykey;
+    key = max(key, dpp_u32<0xB1>(key));  // quad_perm [1,0,3,2]
+    if constexpr (TPR == 2) mykey = key;
+    key = max(key, dpp_u32<0x4E>(key));  // quad_perm [2,3,0,1]
+    if constexpr (TPR == 4) mykey = key;
+    key = max(key, dpp_u32<0x141>(key)); // row_half_mirror
+    key = max(key, dpp_u32<0x140>(key)); // row_mirror
+    if ((threadIdx.x & 15) == 15)           // one lane per 16
+      __hip_atomic_fetch_max(&sm.key[zero_off + (c & 3)], key, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+  };
+  // minus its reciprocal, should it win
+  bool zero = false;
+  auto invert = [&](cx<T> x) __attribute__((always_inline)) {
+    T den = x.re * x.re + x.im * x.im;
+    zero = !(den > T(0));
+    if (zero) {
+      x = cx<T>{tiny_pivot<T>(), T(0)};
+      den = x.re * x.re;
+    }
+    const T iden = T(1) / den;
+    return cx<T>{-(x.re * iden), x.im * iden};
+  };
+  compete(v[0], s0);
+  cx<T> ninv = invert(v[0]);
+#pragma unroll
+  for (int c = 0; c < SW; ++c) {
+    if (c < kw) {                       // uniform
+      const int hc = c / CPT, vc = c % CPT;   // where column c is
+      __syncthreads();
+      const bool isp = sm.key[(s0 + c) & 3] == mykey;
+      // only the pivot row's threads store it, behind a second barrier (every
+      // wave storing its best candidate beside its key costs more)
+      if (isp) {
+#pragma unroll
+        for (int k = 0; k < CPT; ++k) sm.row[c & 1][CPT * h + k] = v[k];
+        if (h == hc) {
+          sm.inv[c] = ninv;
+          if (zero) sing = min(sing, j0 + c + 1);
+        }
+        role = j0 + c;
+        rk = mk = 0;
+      }
+      __syncthreads();
+      const cx<T> pinv = sm.inv[c];
+      cx<T> u[CPT];
+#pragma unroll
+      for (int k = 0; k < CPT; ++k) u[k] = sm.row[c & 1][CPT * h + k];
+      cx<T> x = v[vc];
+      // the row's entry in column c, from the lane that holds it
+      if constexpr (TPR == 2) x = hc == 0 ? dpp_cx<0xA0>(x) : dpp_cx<0xF5>(x);   // quad_perm [0,0,2,2], [1,1,3,3]
+      if constexpr (TPR == 4)
+        x = hc == 0 ? dpp_cx<0x00>(x) : hc == 1 ? dpp_cx<0x55>(x) : hc == 2 ? dpp_cx<0xAA>(x) : dpp_cx<0xFF>(x);
+      // Rows past n and columns past w hold zeros (and the pivot row's copy
+      // too), so the update needs no row or column guard: zeros stay zeros.
+      // The pivot row is not scaled here: its column c becomes 1 and the row
+      // is multiplied by its inverse pivot once, after the last step (a later
+      // step updates it like any other row, which commutes with that scale).
+      // So every lane runs the same code, the pivot row with multiplier zero.
+      cx<T> nl = cmul(x, pinv);
+      if (isp) nl = czero<T>();
+      const cx<T> fin{isp ? T(1) : nl.re, nl.im};
+      // the next pivot column first: its key is the next link of the chain,
+      // and the other columns' updates and the reciprocal run behind it
+      const int hn = (c + 1) / CPT, vn = (c + 1) % CPT;
+      if (c + 1 < SW) {
+        const cx<T> t = ONCE ? cadd(v[vn], cmul_fma(nl, u[vn])) : cfma(v[vn], nl, u[vn]);
+        v[vn] = vn == vc && h == hc ? fin : t;
+        if (TPR > 1 && vn == 0) {       // the columns of the next lane slice begin
+          rk = role == -1 && h == hn ? rowkey : 0u;
+          mk = role == -1 && h == hn ? 0x7FFFFE00u : 0u;
+        }
+        if (c + 1 < kw) compete(v[vn], s0 + c + 1);
+      }
+      if (threadIdx.x == 0) sm.key[(s0 + c + 2) & 3] = 0;      // last read two steps ago, next written in the next step
+#pragma unroll
+      for (int k = 0; k < CPT; ++k)
+        if (k != vn || c + 1 == SW) {
+          const cx<T> t = ONCE ? cadd(v[k], cmul_fma(nl, u[k])) : cfma(v[k], nl, u[k]);
+          v[k] = k == vc && h == hc ? fin : t;
+        }
+      if (c + 1 < SW) ninv = invert(v[vn]);
+    }
+  }
+  const int kp = role >= j0 ? role - (j0) : -1;   // pivot row of these columns: which one
+  if (kp >= 0) {                        // the deferred scale
+    const cx<T> ip{-sm.inv[kp].re, -sm.inv[kp].im};
+    if (h == 0) sm.piv[s0 + kp] = r;
+#pragma unroll
+    for (int k = 0; k < CPT; ++k) v[k] = cmul(v[k], ip);
+  }
+  return kp;
+}
+
 template <class T, int NMAX>
 __global__ __launch_bounds__((NMAX * GJ_TPR<T, NMAX>), (sizeof(T) == 4 ? 4 : 2)) void gj_panel_kernel(
     const InvDesc<T>* __restrict__ descs, int p0) {
@@ -383,11 +511,7 @@ __global__ __launch_bounds__((NMAX * GJ_TPR<T, NMAX>), (sizeof(T) == 4 ? 4 : 2))
   static_assert(WP == 32 && SW == 8, "panel split");
   __shared__ cx<T> sX[SW * LX];           // eliminated columns, row by row: column k of row r at k LX + r
   __shared__ cx<T> sR[SW * WP];           // pivot rows before the update
-  __shared__ cx<T> sRow[2][SW];           // the pivot row
-  __shared__ cx<T> sInv[SW];              // minus the inverse pivots
-  __shared__ unsigned sKey[4];            // best key of a step; steps take the four in turn
-  __shared__ int sPiv[WP];
-  __shared__ int sSing;
+  __shared__ GjLds<T, SW> sm;
   const InvDesc<T> d = descs[blockIdx.x];
   const int n = d.n;
   if (p0 >= n) return;                    // uniform: this block is already done
@@ -426,9 +550,9 @@ __global__ __launch_bounds__((NMAX * GJ_TPR<T, NMAX>), (sizeof(T) == 4 ? 4 : 2))
   int zero_off = 0;
   asm("" : "+v"(zero_off));
   int sing = INT_MAX;                     // smallest singular column (1-based) that this thread has met
-  if (tid == 0) sSing = INT_MAX;
-  if (tid < 4) sKey[tid] = 0;
-  if (tid < WP) sPiv[tid] = 0;
+  if (tid == 0) sm.sing = INT_MAX;
+  if (tid < 4) sm.key[tid] = 0;
+  if (tid < WP) sm.piv[tid] = 0;
   __syncthreads();
   int q0, wo;
   gj_outer_range(n, p0, q0, wo);
@@ -440,7 +564,7 @@ __global__ __launch_bounds__((NMAX * GJ_TPR<T, NMAX>), (sizeof(T) == 4 ? 4 : 2))
   cx<T> gx[GP];
   const int gk = tid % SW, gj = tid / SW;
   auto gather = [&](int s0) __attribute__((always_inline)) {
-    const cx<T>* row = M + sPiv[s0 + gk] + (int64_t)q0 * ld;
+    const cx<T>* row = M + sm.piv[s0 + gk] + (int64_t)q0 * ld;
 #pragma unroll
     for (int t = 0; t < GP; ++t) gx[t] = gld(row + (int64_t)min(gj + t * GC, wo - 1) * ld);
     for (int j = gj + GP * GC; j < wo; j += GC) gst(R + (int64_t)(q0 + j) * WP + s0 + gk, gld(row + (int64_t)j * ld));
@@ -501,107 +625,7 @@ __global__ __launch_bounds__((NMAX * GJ_TPR<T, NMAX>), (sizeof(T) == 4 ? 4 : 2))
     cx<T> v[CPT];
 #pragma unroll
     for (int k = 0; k < CPT; ++k) v[k] = sX[(CPT * h + k) * LX + r];
-    // A step's key is one mask and one or: rows in use have both zero.  Every
-    // column has an unused row left, so the best key is never zero.
-    const unsigned rowkey = 0x80000000u | (unsigned)(511 - r);
-    unsigned rk = role == -1 && h == 0 ? rowkey : 0u, mk = role == -1 && h == 0 ? 0x7FFFFE00u : 0u;
-    unsigned mykey = 0;                   // of the row (of both its lanes)
-    // the row's entry x of column s0 + c enters the search for its pivot
-    auto compete = [&](cx<T> x, int c) __attribute__((always_inline)) {
-      mykey = (pivot_bits(cabs1(x)) & mk) | rk;
-      unsigned key = mykey;
-      key = max(key, dpp_u32<0xB1>(key));  // quad_perm [1,0,3,2]
-      if constexpr (TPR == 2) mykey = key;
-      key = max(key, dpp_u32<0x4E>(key));  // quad_perm [2,3,0,1]
-      key = max(key, dpp_u32<0x141>(key)); // row_half_mirror
-      key = max(key, dpp_u32<0x140>(key)); // row_mirror
-      if (l16 == 15) __hip_atomic_fetch_max(&sKey[zero_off + (c & 3)], key, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-    };
-    // minus its reciprocal, should it win
-    bool zero = false;
-    auto invert = [&](cx<T> x) __attribute__((always_inline)) {
-      T den = x.re * x.re + x.im * x.im;
-      zero = !(den > T(0));
-      if (zero) {
-        x = cx<T>{tiny_pivot<T>(), T(0)};
-        den = x.re * x.re;
-      }
-      const T iden = T(1) / den;
-      return cx<T>{-(x.re * iden), x.im * iden};
-    };
-    compete(v[0], s0);
-    cx<T> ninv = invert(v[0]);
-#pragma unroll
-    for (int c = 0; c < SW; ++c) {
-      if (c < kw) {                       // uniform
-        const int hc = c / CPT, vc = c % CPT;   // where column c is
-        __syncthreads();
-        const bool isp = sKey[(s0 + c) & 3] == mykey;
-        // only the pivot row's threads store it, behind a second barrier (every
-        // wave storing its best candidate beside its key costs more)
-        if (isp) {
-#pragma unroll
-          for (int k = 0; k < CPT; ++k) sRow[c & 1][CPT * h + k] = v[k];
-          if (h == hc) {
-            sInv[c] = ninv;
-            if (zero) sing = min(sing, p0 + s0 + c + 1);
-          }
-          role = p0 + s0 + c;
-          rk = mk = 0;
-        }
-        __syncthreads();
-        const cx<T> pinv = sInv[c];
-        cx<T> u[CPT];
-#pragma unroll
-        for (int k = 0; k < CPT; ++k) u[k] = sRow[c & 1][CPT * h + k];
-        cx<T> x = v[vc];
-        if constexpr (TPR == 2) {         // the row's entry in column c, from the lane that holds it
-          if (hc == 0) {
-            x.re = dpp_t<0xA0>(x.re);     // quad_perm [0,0,2,2]
-            x.im = dpp_t<0xA0>(x.im);
-          } else {
-            x.re = dpp_t<0xF5>(x.re);     // quad_perm [1,1,3,3]
-            x.im = dpp_t<0xF5>(x.im);
-          }
-        }
-        // Rows past n and columns past w hold zeros (and the pivot row's copy
-        // too), so the update needs no row or column guard: zeros stay zeros.
-        // The pivot row is not scaled here: its column c becomes 1 and the row
-        // is multiplied by its inverse pivot once, after the last step (a later
-        // step updates it like any other row, which commutes with that scale).
-        // So every lane runs the same code, the pivot row with multiplier zero.
-        cx<T> nl = cmul(x, pinv);
-        if (isp) nl = czero<T>();
-        const cx<T> fin{isp ? T(1) : nl.re, nl.im};
-        // the next pivot column first: its key is the next link of the chain,
-        // and the other columns' updates and the reciprocal run behind it
-        const int hn = (c + 1) / CPT, vn = (c + 1) % CPT;
-        if (c + 1 < SW) {
-          const cx<T> t = cfma(v[vn], nl, u[vn]);
-          v[vn] = vn == vc && h == hc ? fin : t;
-          if (TPR == 2 && vn == 0) {      // the columns of the other lane slice begin
-            rk = role == -1 && h == hn ? rowkey : 0u;
-            mk = role == -1 && h == hn ? 0x7FFFFE00u : 0u;
-          }
-          if (c + 1 < kw) compete(v[vn], s0 + c + 1);
-        }
-        if (tid == 0) sKey[(s0 + c + 2) & 3] = 0;      // last read two steps ago, next written in the next step
-#pragma unroll
-        for (int k = 0; k < CPT; ++k)
-          if (k != vn || c + 1 == SW) {
-            const cx<T> t = cfma(v[k], nl, u[k]);
-            v[k] = k == vc && h == hc ? fin : t;
-          }
-        if (c + 1 < SW) ninv = invert(v[vn]);
-      }
-    }
-    const int kp = role >= p0 + s0 ? role - (p0 + s0) : -1;   // pivot row of these columns: which one
-    if (kp >= 0) {                        // the deferred scale
-      const cx<T> ip{-sInv[kp].re, -sInv[kp].im};
-      if (h == 0) sPiv[s0 + kp] = r;
-#pragma unroll
-      for (int k = 0; k < CPT; ++k) v[k] = cmul(v[k], ip);
-    }
+    const int kp = gj_eliminate<T, SW, TPR, false>(sm, v, role, sing, p0 + s0, s0, kw, zero_off);
 #pragma unroll
     for (int k = 0; k < CPT; ++k) sX[(CPT * h + k) * LX + r] = v[k];
     // the pivot rows' other columns go to sR and are cleared: the product then
@@ -646,17 +670,93 @@ __global__ __launch_bounds__((NMAX * GJ_TPR<T, NMAX>), (sizeof(T) == 4 ? 4 : 2))
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           const int j = 16 * ct + 4 * i + lq;
-          if (j < w) gst(whole ? d.scratch + sPiv[j] * n + to : J + j * ld + row, cx<T>{cre[rt][ct][i], cim[rt][ct][i]});
+          if (j < w) gst(whole ? d.scratch + sm.piv[j] * n + to : J + j * ld + row, cx<T>{cre[rt][ct][i], cim[rt][ct][i]});
         }
     }
   }
   if (live && h == 0 && !whole) roles[r] = role;
-  if (tid < w) d.ipiv[p0 + tid] = sPiv[tid];
+  if (tid < w) d.ipiv[p0 + tid] = sm.piv[tid];
   // info: reset by the first panel, then the first singular column wins
-  if (sing != INT_MAX) atomicMin(&sSing, sing);
+  if (sing != INT_MAX) atomicMin(&sm.sing, sing);
   __syncthreads();
   if (tid == 0 && d.info) {
-    const int col = sSing == INT_MAX ? 0 : sSing;
+    const int col = sm.sing == INT_MAX ? 0 : sm.sing;
+    if (p0 == 0 || (col && *d.info == 0)) *d.info = col;
+  }
+}
+
+// The same for blocks of up to NMAX = 64 rows: four threads per row hold all 32
+// columns of the panel, so that every column is eliminated one by one.  Eight at a
+// time, as above, cost these blocks accuracy (mean residual of A A^{-1} over 150
+// complex128 blocks: 24 rows 2.5e-15 against 2.1e-15, 48 rows 5.3e-15 against 4.5e-15; 100
+// rows 1.35e-14 against 1.29e-14, from 200 rows on there is no difference) and time, since
+// there is little to take off the chain (64 rows 63 against 60 us, complex64 57
+// against 50); with 128 rows this form is the slower one (130 against 158 us).
+template <class T, int NMAX>
+__global__ __launch_bounds__(4 * NMAX) void gj_panel_rows_kernel(const InvDesc<T>* __restrict__ descs, int p0) {
+  constexpr int WP = GJM_WP, TPR = 4, CPT = WP / TPR, NT = 4 * NMAX;
+  __shared__ GjLds<T, WP> sm;
+  const InvDesc<T> d = descs[blockIdx.x];
+  const int n = d.n;
+  if (p0 >= n) return;                    // uniform: this block is already done
+  const int64_t ld = d.ld;
+  cx<T>* __restrict__ M = d.M;
+  cx<T>* __restrict__ R = d.scratch;
+  int* __restrict__ roles = reinterpret_cast<int*>(d.scratch + (size_t)WP * n);
+  const int w = min(WP, n - p0);
+  const int tid = threadIdx.x, r = tid / TPR, h = tid % TPR;
+  const bool live = r < n;
+  cx<T>* J = M + (int64_t)p0 * ld;
+  cx<T> v[CPT];
+#pragma unroll
+  for (int k = 0; k < CPT; ++k) {
+    const int j = CPT * h + k;
+    v[k] = gld_at<T>(J, (unsigned)min(j, w - 1) * (unsigned)ld + (unsigned)min(r, n - 1));
+    if (!live || j >= w) v[k] = czero<T>();
+  }
+  int role = -2;
+  if (live) role = p0 == 0 ? -1 : roles[r];
+  int zero_off = 0;                       // see gj_panel_kernel
+  asm("" : "+v"(zero_off));
+  int sing = INT_MAX;
+  if (tid == 0) sm.sing = INT_MAX;
+  if (tid < 4) sm.key[tid] = 0;
+  if (tid < WP) sm.piv[tid] = 0;
+  __syncthreads();
+  gj_eliminate<T, WP, TPR, true>(sm, v, role, sing, p0, 0, w, zero_off);
+  __syncthreads();                        // all pivot rows are in sm.piv
+  // C -> M[:, J]; a block of one panel goes to its place in its final order,
+  // A^{-1}[k, l] = C[r_k, r^{-1}(l)]
+  const bool whole = n <= WP;
+  if (live) {
+#pragma unroll
+    for (int k = 0; k < CPT; ++k) {
+      const int j = CPT * h + k;
+      if (j < w) gst(whole ? d.scratch + sm.piv[j] * n + role : J + j * ld + r, v[k]);
+    }
+    if (h == 0 && !whole) roles[r] = role;
+  }
+  if (tid < w) d.ipiv[p0 + tid] = sm.piv[tid];
+  // R[k, j] = M[P[k], j] for the columns j outside the panel (rows k from w on repeat
+  // row 0's place and are not used)
+  if (!whole) {
+    const int k = tid % WP;
+    const cx<T>* row = M + sm.piv[k];
+    constexpr int CS = NT / WP, RB = NMAX / CS;
+    cx<T> x[RB];
+#pragma unroll
+    for (int t = 0; t < RB; ++t) x[t] = gld(row + (int64_t)min(tid / WP + t * CS, n - 1) * ld);
+#pragma unroll
+    for (int t = 0; t < RB; ++t) {
+      const int j = tid / WP + t * CS;
+      if (j < n && (j < p0 || j >= p0 + w)) gst(R + (int64_t)j * WP + k, x[t]);
+    }
+  }
+  // info: reset by the first panel, then the first singular column wins
+  if (sing != INT_MAX) atomicMin(&sm.sing, sing);
+  __syncthreads();
+  if (tid == 0 && d.info) {
+    const int col = sm.sing == INT_MAX ? 0 : sm.sing;
     if (p0 == 0 || (col && *d.info == 0)) *d.info = col;
   }
 }
@@ -831,7 +931,7 @@ static hipError_t gj_inverse_launches(const InvDesc<T>* d_descs, int ndesc, int 
   const int nt = (nmax + 63) / 64;
   for (int p0 = 0; p0 < nmax; p0 += GJM_WP) {
     if (nmax <= 64)
-      hipLaunchKernelGGL((gj_panel_kernel<T, 64>), dim3(ndesc), dim3(64 * GJ_TPR<T, 64>), 0, s, d_descs, p0);
+      hipLaunchKernelGGL((gj_panel_rows_kernel<T, 64>), dim3(ndesc), dim3(4 * 64), 0, s, d_descs, p0);
     else if (nmax <= 128)
       hipLaunchKernelGGL((gj_panel_kernel<T, 128>), dim3(ndesc), dim3(128 * GJ_TPR<T, 128>), 0, s, d_descs, p0);
     else if (nmax <= 256)

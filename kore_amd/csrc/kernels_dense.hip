@@ -670,7 +670,8 @@ __global__ __launch_bounds__((NMAX * GJ_TPR<T, NMAX>), (sizeof(T) == 4 ? 4 : 2))
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           const int j = 16 * ct + 4 * i + lq;
-          if (j < w) gst(whole ? d.scratch + sm.piv[j] * n + to : J + j * ld + row, cx<T>{cre[rt][ct][i], cim[rt][ct][i]});
+          cx<T>* at = whole ? d.scratch + sm.piv[j] * n + to : J + j * ld + row;
+          if (j < w) gst(at, cx<T>{cre[rt][ct][i], cim[rt][ct][i]});
         }
     }
   }

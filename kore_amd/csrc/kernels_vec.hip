@@ -449,7 +449,8 @@ __global__ __launch_bounds__(256) void skinny_kernel(const SkinnyDesc<T>* __rest
 // 257 to 512 rows fit the registers and cost one memory round trip.
 constexpr int SKD_KS = 32;
 template <class T, int NR>
-__global__ __launch_bounds__(SK_ROWS * SKD_KS) void skinny_deep_kernel(const SkinnyDesc<T>* __restrict__ descs, int nrhs) {
+__global__ __launch_bounds__(SK_ROWS * SKD_KS) void skinny_deep_kernel(const SkinnyDesc<T>* __restrict__ descs,
+                                                                      int nrhs) {
   const SkinnyDesc<T>& d = descs[blockIdx.y];
   const int r0 = blockIdx.x * SK_ROWS;
   if (r0 >= d.m) return;

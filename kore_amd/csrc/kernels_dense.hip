@@ -370,7 +370,7 @@ __device__ __forceinline__ unsigned pivot_bits(float mag) {
 constexpr int GJ_SW = 8;
 template <class T, int NMAX> constexpr int GJ_TPR = sizeof(T) == 8 && NMAX > 256 ? 1 : 2;
 // columns of a pivot row that a panel keeps in flight: all of an outer panel's
-constexpr int gj_gather_cols(int nmax) { return nmax <= 256 ? nmax : 128; }
+constexpr int gj_gather_cols(int nmax) { return nmax <= 256 ? nmax : nmax <= 384 ? 192 : 128; }
 
 template <class T> __device__ __forceinline__ cx<T> cmul_fma(cx<T> a, cx<T> b) {
   return cx<T>{fma(a.re, b.re, -(a.im * b.im)), fma(a.re, b.im, a.im * b.re)};
@@ -931,12 +931,20 @@ template <class T>
 static hipError_t gj_inverse_launches(const InvDesc<T>* d_descs, int ndesc, int nmax, hipStream_t s) {
   const int nt = (nmax + 63) / 64;
   for (int p0 = 0; p0 < nmax; p0 += GJM_WP) {
+    // the smallest workgroup that has the rows: fewer waves meet at a step's barriers
+    // (an inversion of one block: complex64 300 rows, 384 instead of 512, 424 -> 388 us,
+    // 374 rows 520 -> 477; complex128 150 rows, 192 instead of 256, 194 -> 189)
     if (nmax <= 64)
       hipLaunchKernelGGL((gj_panel_rows_kernel<T, 64>), dim3(ndesc), dim3(4 * 64), 0, s, d_descs, p0);
     else if (nmax <= 128)
       hipLaunchKernelGGL((gj_panel_kernel<T, 128>), dim3(ndesc), dim3(128 * GJ_TPR<T, 128>), 0, s, d_descs, p0);
+    else if (nmax <= 192)
+      hipLaunchKernelGGL((gj_panel_kernel<T, 192>), dim3(ndesc), dim3(192 * GJ_TPR<T, 192>), 0, s, d_descs, p0);
     else if (nmax <= 256)
       hipLaunchKernelGGL((gj_panel_kernel<T, 256>), dim3(ndesc), dim3(256 * GJ_TPR<T, 256>), 0, s, d_descs, p0);
+    else if (sizeof(T) == 4 && nmax <= 384)
+      hipLaunchKernelGGL((gj_panel_kernel<float, 384>), dim3(ndesc), dim3(384 * GJ_TPR<float, 384>), 0, s,
+                         reinterpret_cast<const InvDesc<float>*>(d_descs), p0);
     else
       hipLaunchKernelGGL((gj_panel_kernel<T, 512>), dim3(ndesc), dim3(512 * GJ_TPR<T, 512>), 0, s, d_descs, p0);
     if (nmax <= GJM_WP) return hipGetLastError();          // one panel, stored in its final order

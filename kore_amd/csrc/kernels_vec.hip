@@ -534,20 +534,25 @@ template hipError_t launch_skinny1<double>(const SkinnyDesc<double>&, int, hipSt
 
 // Three and more right-hand sides: Y = beta Y + sum_p alpha_p A_p X_p on the matrix
 // cores, 16 rows by 16 columns per workgroup (unused columns repeat the last).
-// The k of a product stand in groups of four, which the NW waves take in turn:
+// The k of a product stand in groups of four, which the eight waves take in turn:
 // lane (lq, l16) loads A[r0 + l16][4 g + lq] (16 lanes read 256 consecutive bytes)
 // and X[4 g + lq][l16] straight into registers, SKM_NB groups requested before the
 // first is used; the waves' sums are added through LDS.  Bound by the memory
 // round trips on few blocks and by reading A (with X from L2) on many.
-// Measured against the vector kernel, us per launch of complex128 products of
-// 200 rows: 16 columns, 150 blocks 102 -> 35 (one product each) and 162 -> 67
-// (two), one block 19 -> 7 and 30 -> 11; 8 columns 47 -> 32 and 78 -> 58, one block
-// 18 -> 10.  Eight waves instead of four: no faster on one block, 40 and 69 us on 150.
-constexpr int SKM_NB = 8;
+// An accumulator adds every k of its groups one after the other, so the split also
+// sets the error: eight waves and the four real products in accumulators of their
+// own add K / 8 terms each, as the vector kernel's threads do.  Root mean square error of
+// random operands, over the vector kernel's: 0.73 to 0.99 (24 to 500 rows, both
+// types); with four waves and two accumulators it was 1.3 at one block of 24 rows and 1.88 at
+// 500.  Measured against the vector kernel and against four waves of eight groups, us per
+// launch of two complex128 products of 200 rows, 16 columns: one block 28.2 / 10.0 /
+// 8.6, 150 blocks 151 / 57.7 / 57.0; eight waves of eight groups 9.8 and 78.
+constexpr int SKM_NB = 4, SKM_NW = 8;
 
-template <class T, int NW>
-__global__ __launch_bounds__(64 * NW) void skinny_mm_kernel(const SkinnyDesc<T>* __restrict__ descs, int nrhs) {
+template <class T>
+__global__ __launch_bounds__(64 * SKM_NW) void skinny_mm_kernel(const SkinnyDesc<T>* __restrict__ descs, int nrhs) {
   using A4 = typename acc4<T>::type;
+  constexpr int NW = SKM_NW;
   const SkinnyDesc<T>& d = descs[blockIdx.y];   // read in place (uniform loads, no private copy)
   const int r0 = blockIdx.x * SK_ROWS;
   if (r0 >= d.m) return;
@@ -557,7 +562,7 @@ __global__ __launch_bounds__(64 * NW) void skinny_mm_kernel(const SkinnyDesc<T>*
   const int l16 = lane & 15, lq = lane >> 4;
   const int rc = min(r0 + l16, d.m - 1);        // rows past the block repeat its last one (not stored)
   const int xc = min(l16, nrhs - 1);
-  A4 cre = {0, 0, 0, 0}, cim = {0, 0, 0, 0};
+  A4 rr = {0, 0, 0, 0}, ii = {0, 0, 0, 0}, ri = {0, 0, 0, 0}, ir = {0, 0, 0, 0};
 #pragma unroll 1
   for (int p = 0; p < 3; ++p) {
     const int K = d.A[p] != nullptr ? d.k[p] : 0;
@@ -585,9 +590,16 @@ __global__ __launch_bounds__(64 * NW) void skinny_mm_kernel(const SkinnyDesc<T>*
         }
       }
 #pragma unroll
-      for (int t = 0; t < SKM_NB; ++t) cmma<T>(cre, cim, a[t], cx<T>{al * x[t].re, al * x[t].im});
+      for (int t = 0; t < SKM_NB; ++t) {
+        const T xre = al * x[t].re, xim = al * x[t].im;
+        rr = mfma16(xre, a[t].re, rr);
+        ii = mfma16(xim, a[t].im, ii);
+        ri = mfma16(xim, a[t].re, ri);
+        ir = mfma16(xre, a[t].im, ir);
+      }
     }
   }
+  const A4 cre = rr - ii, cim = ri + ir;
 #pragma unroll
   for (int i = 0; i < 4; ++i) sP[wave][mfma_mrow<T>(lq, i)][l16] = cx<T>{cre[i], cim[i]};
   __syncthreads();
@@ -770,7 +782,7 @@ hipError_t launch_skinny(const SkinnyDesc<T>* d_descs, int ndesc, int max_m, int
   else if (nrhs <= 4 && max_m > 128 && max_m <= 256)
     hipLaunchKernelGGL((skinny_kernel<T, 4>), grid, dim3(256), 0, s, d_descs, nrhs);
   else
-    hipLaunchKernelGGL((skinny_mm_kernel<T, 4>), grid, dim3(256), 0, s, d_descs, nrhs);
+    hipLaunchKernelGGL(skinny_mm_kernel<T>, grid, dim3(64 * SKM_NW), 0, s, d_descs, nrhs);
   return hipGetLastError();
 }
 template hipError_t launch_skinny<double>(const SkinnyDesc<double>*, int, int, int, hipStream_t);

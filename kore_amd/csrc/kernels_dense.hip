@@ -44,7 +44,8 @@ template <class T> __device__ __forceinline__ cx<T> gld_at(const cx<T>* base, un
 // that only the last slab of a product has anything to check: its missing k
 // count as zero.  With roles given, rows of C whose role is rmin or more are
 // replaced (their old values count as zero).
-template <class T, int S>
+// M3: three real products per complex step in complex64 (below).
+template <class T, int S, bool M3 = true>
 __device__ __forceinline__ void gemm_tile_body(const GemmDesc<T>& d, const int tile, GemmLds<T, S>& sm,
                                                const int* roles = nullptr, int rmin = 0) {
   using A4 = typename acc4<T>::type;
@@ -77,7 +78,7 @@ __device__ __forceinline__ void gemm_tile_body(const GemmDesc<T>& d, const int t
   // form makes the FP64 factor 10 % faster at N = 500 but moves the most
   // ill-conditioned MAC eigenvalues (relative condition 1e16) further from
   // the oracle's than the four-product form does.
-  constexpr bool k3m = sizeof(T) == 4;
+  constexpr bool k3m = M3 && sizeof(T) == 4;
   A4 cre[S][S], cim[S][S], csum[S][S];
 #pragma unroll
   for (int a = 0; a < S; ++a)
@@ -606,9 +607,13 @@ __global__ __launch_bounds__((NMAX * GJ_TPR<T, NMAX>), (sizeof(T) == 4 ? 4 : 2))
 #pragma unroll
       for (int k = 0; k < NK; ++k) a[k] = sX[(4 * k + lq) * LX + RW * wave + 16 * rt + l16];
 #pragma unroll
-      for (int ct = 0; ct < 2; ++ct)
+      for (int ct = 0; ct < 2; ++ct) {        // the product on its own, added once: each entry rounds once
+        A4 pre = {0, 0, 0, 0}, pim = {0, 0, 0, 0};
 #pragma unroll
-        for (int k = 0; k < NK; ++k) cmma<T>(cre[rt][ct], cim[rt][ct], a[k], b[ct][k]);
+        for (int k = 0; k < NK; ++k) cmma<T>(pre, pim, a[k], b[ct][k]);
+        cre[rt][ct] += pre;
+        cim[rt][ct] += pim;
+      }
 #pragma unroll
       for (int k = 0; k < NK; ++k) {
         cre[rt][CT][I0 + k] = a[k].re;
@@ -625,7 +630,7 @@ __global__ __launch_bounds__((NMAX * GJ_TPR<T, NMAX>), (sizeof(T) == 4 ? 4 : 2))
     cx<T> v[CPT];
 #pragma unroll
     for (int k = 0; k < CPT; ++k) v[k] = sX[(CPT * h + k) * LX + r];
-    const int kp = gj_eliminate<T, SW, TPR, false>(sm, v, role, sing, p0 + s0, s0, kw, zero_off);
+    const int kp = gj_eliminate<T, SW, TPR, NMAX <= 128>(sm, v, role, sing, p0 + s0, s0, kw, zero_off);
 #pragma unroll
     for (int k = 0; k < CPT; ++k) sX[(CPT * h + k) * LX + r] = v[k];
     // the pivot rows' other columns go to sR and are cleared: the product then
@@ -686,13 +691,18 @@ __global__ __launch_bounds__((NMAX * GJ_TPR<T, NMAX>), (sizeof(T) == 4 ? 4 : 2))
   }
 }
 
-// The same for blocks of up to NMAX = 64 rows: four threads per row hold all 32
-// columns of the panel, so that every column is eliminated one by one.  Eight at a
-// time, as above, cost these blocks accuracy (mean residual of A A^{-1} over 150
-// complex128 blocks: 24 rows 2.5e-15 against 2.1e-15, 48 rows 5.3e-15 against 4.5e-15; 100
-// rows 1.35e-14 against 1.29e-14, from 200 rows on there is no difference) and time, since
-// there is little to take off the chain (64 rows 63 against 60 us, complex64 57
-// against 50); with 128 rows this form is the slower one (130 against 158 us).
+// The same for blocks of up to GJ_ROWS_MAX rows: four threads per row hold all 32 columns of
+// the panel, so that every column is eliminated one by one.  Eight at a time, as
+// above, cost these blocks accuracy.  Residual of A A^{-1} (geometric mean over 400
+// random blocks and more), over that of one column at a time with every step rounded once:
+// complex128 65 rows 1.15, 74 rows 1.11, 95 rows 1.11; with the product of eight added once
+// and its steps rounded once (the 128-row instance above) still 1.11, 1.06 and 1.06, and 1.01
+// at 97 rows over the earlier panel kernel, which updated all 32 columns by fused
+// multiply-adds; from 104 rows on 0.99.  This form: 0.99 to 1.00, and 0.95 at 96 to 112 rows.
+// Up to 64 rows it is the faster one too (64 rows 59 against 63 us, complex64 51 against 57);
+// above it costs a tenth: 74 rows 84 -> 90 us, 95 rows 100 -> 112, 112 rows 120 -> 142 in
+// complex128, 74 -> 78, 87 -> 94 and 106 -> 118 in complex64.
+constexpr int GJ_ROWS_MAX = 112;
 template <class T, int NMAX>
 __global__ __launch_bounds__(4 * NMAX) void gj_panel_rows_kernel(const InvDesc<T>* __restrict__ descs, int p0) {
   constexpr int WP = GJM_WP, TPR = 4, CPT = WP / TPR, NT = 4 * NMAX;
@@ -766,7 +776,10 @@ __global__ __launch_bounds__(4 * NMAX) void gj_panel_rows_kernel(const InvDesc<T
 // outer panel outside J, the pivot rows' old values counting as zero, on the
 // batched GEMM's tile with descriptors made here (columns [q0, p0), then
 // [p0 + w, q0 + wo)); K = w <= 32.
-template <class T, int S>
+// M3 = false up to GJ_ROWS_MAX rows: the 3M product's error (relative to the product of
+// the norms and not entry by entry) shows there, residual of complex64 inverses over that of four
+// products 1.04 at 48 and 64 rows, 1.09 at 74 and 95, 1.12 at 112.
+template <class T, int S, bool M3>
 __global__ __launch_bounds__(256, 3) void gj_update_kernel(const InvDesc<T>* __restrict__ descs, int ndesc, int per,
                                                            int p0) {
   constexpr int TS = 32 * S;
@@ -804,7 +817,7 @@ __global__ __launch_bounds__(256, 3) void gj_update_kernel(const InvDesc<T>* __r
   d.n = ncols;
   d.alpha = T(1);
   d.beta = T(1);
-  gemm_tile_body<T, S>(d, t, sm, reinterpret_cast<const int*>(v.scratch + (size_t)GJM_WP * n), p0);
+  gemm_tile_body<T, S, M3>(d, t, sm, reinterpret_cast<const int*>(v.scratch + (size_t)GJM_WP * n), p0);
 }
 
 // S[l n + k] = M[r_k, r^{-1}(l)], the inverse in its final order and place.  Grid:
@@ -917,7 +930,12 @@ static void launch_gj_updates(const InvDesc<T>* d_descs, int ndesc, int nmax, in
   // GJ_OUTER_MIN rows (whichever is more when a launch holds both)
   const int ntb = ((nmax < GJ_OUTER_MIN ? nmax : GJ_OUTER_MIN) + TS - 1) / TS + 1;
   const int per = nt * (nmax >= GJ_OUTER_MIN && ntb < GJ_WO / TS + 1 ? GJ_WO / TS + 1 : ntb);
-  hipLaunchKernelGGL((gj_update_kernel<T, S>), dim3(xcd_grid(ndesc, per)), dim3(256), 0, s, d_descs, ndesc, per, p0);
+  if (sizeof(T) == 4 && nmax <= GJ_ROWS_MAX)
+    hipLaunchKernelGGL((gj_update_kernel<T, S, false>), dim3(xcd_grid(ndesc, per)), dim3(256), 0, s, d_descs, ndesc,
+                       per, p0);
+  else
+    hipLaunchKernelGGL((gj_update_kernel<T, S, true>), dim3(xcd_grid(ndesc, per)), dim3(256), 0, s, d_descs, ndesc,
+                       per, p0);
 }
 
 template <class T, int S>
@@ -936,6 +954,10 @@ static hipError_t gj_inverse_launches(const InvDesc<T>* d_descs, int ndesc, int 
     // 374 rows 520 -> 477; complex128 150 rows, 192 instead of 256, 194 -> 189)
     if (nmax <= 64)
       hipLaunchKernelGGL((gj_panel_rows_kernel<T, 64>), dim3(ndesc), dim3(4 * 64), 0, s, d_descs, p0);
+    else if (nmax <= 96)
+      hipLaunchKernelGGL((gj_panel_rows_kernel<T, 96>), dim3(ndesc), dim3(4 * 96), 0, s, d_descs, p0);
+    else if (nmax <= GJ_ROWS_MAX)
+      hipLaunchKernelGGL((gj_panel_rows_kernel<T, GJ_ROWS_MAX>), dim3(ndesc), dim3(4 * GJ_ROWS_MAX), 0, s, d_descs, p0);
     else if (nmax <= 128)
       hipLaunchKernelGGL((gj_panel_kernel<T, 128>), dim3(ndesc), dim3(128 * GJ_TPR<T, 128>), 0, s, d_descs, p0);
     else if (nmax <= 192)

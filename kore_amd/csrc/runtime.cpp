@@ -28,6 +28,7 @@
 
 #include <sched.h>
 
+#include "host_parts.hpp"
 #include "kore_amd.h"
 #include "kore_device.hpp"
 #include "kore_kernels.hpp"
@@ -468,15 +469,8 @@ static void copy_parallel(const std::vector<CopySeg>& segs) {
       base += g.bytes;
     }
   };
-  if (nt <= 1) {
-    range(0, total);
-    return;
-  }
   const size_t per = (total + nt - 1) / nt;
-  std::vector<std::thread> th;
-  for (int t = 1; t < nt; ++t) th.emplace_back(range, t * per, std::min(total, (t + 1) * per));
-  range(0, per);
-  for (std::thread& x : th) x.join();
+  run_parts(nt, [&](int t) { range(t * per, std::min(total, (t + 1) * per)); });
 }
 
 // ---------------------------------------------------------------------------
@@ -2205,13 +2199,8 @@ static int32_t sys_prepare(const kore_layout* lay, int64_t sizmat, const int32_t
     tcnt[t] = cntt;
     tcntb[t] = cnttb;
   };
-  {
-    std::vector<std::thread> pool;
-    for (int t = 1; t < nth; ++t) pool.emplace_back(build_rows, t);
-    trace.mark("sys_create checks");
-    build_rows(0);
-    for (auto& th : pool) th.join();
-  }
+  trace.mark("sys_create checks");
+  run_parts(nth, build_rows);
   trace.mark("sys_create union pattern");
   for (int t = 0; t < nth; ++t)
     if (bad_a[t]) return fail(KORE_ERR_ARG, "A: column index out of range");
@@ -2233,10 +2222,7 @@ static int32_t sys_prepare(const kore_layout* lay, int64_t sizmat, const int32_t
           if (s->h_amap[k] >= 0) s->h_amap[k] = (int32_t)(s->h_amap[k] + rbase[t]);
       }
     };
-    std::vector<std::thread> pool;
-    for (int t = 1; t < nth; ++t) pool.emplace_back(fix, t);
-    fix(0);
-    for (auto& th : pool) th.join();
+    run_parts(nth, fix);
   }
   for (int t = 0; t < nth; ++t)
     if (bad_row[t] >= 0)
@@ -2322,11 +2308,8 @@ static int32_t sys_prepare(const kore_layout* lay, int64_t sizmat, const int32_t
           }
         }
     };
-    std::vector<std::thread> pool;
     const int nthb = std::max(1, std::min(nth, s->nblk));
-    for (int t = 1; t < nthb; ++t) pool.emplace_back(fill_blocks, s->nblk * t / nthb, s->nblk * (t + 1) / nthb);
-    fill_blocks(0, s->nblk / nthb);
-    for (auto& th : pool) th.join();
+    run_parts(nthb, [&](int t) { fill_blocks(s->nblk * t / nthb, s->nblk * (t + 1) / nthb); });
   }
   trace.mark("sys_create off-block views");
   return KORE_OK;
@@ -2511,7 +2494,8 @@ int32_t kore_sys_update_a(kore_sys* s, const double* a_data) {
   if (s->a_repeats) std::fill(va, va + s->nnz, zd(0, 0));
   else
     for (int32_t q : s->h_aless) va[q] = zd(0, 0);
-  std::vector<int64_t> bad(nt, -1);       // first entry of each range that has no position and a value
+  int64_t bad[8];                         // first entry of each range that has no position and a value, or -1
+  std::fill(bad, bad + nt, -1);
   auto place = [&](int t) {
     for (int64_t k = na * t / nt; k < na * (t + 1) / nt; ++k) {
       const zd v(a_data[2 * k], a_data[2 * k + 1]);
@@ -2525,12 +2509,7 @@ int32_t kore_sys_update_a(kore_sys* s, const double* a_data) {
       }
     }
   };
-  {
-    std::vector<std::thread> pool;
-    for (int t = 1; t < nt; ++t) pool.emplace_back(place, t);
-    place(0);
-    for (auto& th : pool) th.join();
-  }
+  run_parts(nt, place);
   for (int t = 0; t < nt; ++t)
     if (bad[t] >= 0)
       return fail(KORE_ERR_UNSUPPORTED, "A entry %lld was a zero outside the block-tridiagonal pattern at "

@@ -515,7 +515,7 @@ __global__ __launch_bounds__((NMAX * GJ_TPR<T, NMAX>), (sizeof(T) == 4 ? 4 : 2))
   __shared__ GjLds<T, SW> sm;
   const InvDesc<T> d = descs[blockIdx.x];
   const int n = d.n;
-  if (p0 >= n) return;                    // uniform: this block is already done
+  __builtin_assume(p0 < n);               // no check for an empty panel (complex64, 200 rows: 222 -> 211 us)
   const int64_t ld = d.ld;
   cx<T>* __restrict__ M = d.M;
   cx<T>* __restrict__ R = d.scratch;
@@ -560,15 +560,16 @@ __global__ __launch_bounds__((NMAX * GJ_TPR<T, NMAX>), (sizeof(T) == 4 ? 4 : 2))
   // R[k, j] = M[P[k], j] for the columns j of the outer panel (those of the panel
   // itself are not used): the rows of SW columns are requested as soon as they
   // are known and stored after the next SW columns, behind whose steps the
-  // scattered reads finish.  GP passes of GC columns are kept in flight.
+  // scattered reads finish.  GP passes of GC columns, all of an outer panel's, are
+  // kept in flight.
   constexpr int GC = NT / SW, GP = gj_gather_cols(NMAX) / GC;
+  static_assert(GP * GC >= (NMAX < GJ_OUTER_MIN ? NMAX : GJ_WO), "columns of an outer panel");
   cx<T> gx[GP];
   const int gk = tid % SW, gj = tid / SW;
   auto gather = [&](int s0) __attribute__((always_inline)) {
     const cx<T>* row = M + sm.piv[s0 + gk] + (int64_t)q0 * ld;
 #pragma unroll
     for (int t = 0; t < GP; ++t) gx[t] = gld(row + (int64_t)min(gj + t * GC, wo - 1) * ld);
-    for (int j = gj + GP * GC; j < wo; j += GC) gst(R + (int64_t)(q0 + j) * WP + s0 + gk, gld(row + (int64_t)j * ld));
   };
   auto put = [&](int s0) __attribute__((always_inline)) {
 #pragma unroll
@@ -620,7 +621,8 @@ __global__ __launch_bounds__((NMAX * GJ_TPR<T, NMAX>), (sizeof(T) == 4 ? 4 : 2))
         cim[rt][CT][I0 + k] = a[k].im;
       }
       // the row tiles one after the other: overlapped they take more registers than there
-      // are (complex128, an inversion of one block of 500 rows 933 us instead of 920)
+      // are (complex128, 24 of them spilled, an inversion of one block of 500 rows 961
+      // us instead of 904)
       __builtin_amdgcn_sched_barrier(0);
     }
   };
@@ -665,25 +667,20 @@ __global__ __launch_bounds__((NMAX * GJ_TPR<T, NMAX>), (sizeof(T) == 4 ? 4 : 2))
   eliminate(std::integral_constant<int, 2>{});
   eliminate(std::integral_constant<int, 3>{});
   if (wo > w) put((w - 1) / SW * SW);
-  // C -> M[:, J]; a block of one panel is then complete and is stored in its
-  // final order, A^{-1}[k, l] = C[r_k, r^{-1}(l)]
-  const bool whole = n <= WP;
 #pragma unroll
-  for (int rt = 0; rt < NRT; ++rt) {
+  for (int rt = 0; rt < NRT; ++rt) {      // C -> M[:, J]
     const int row = RW * wave + 16 * rt + l16;
-    const int to = __shfl(role, (16 * rt + l16) * TPR, 64);
     if (row < n) {
 #pragma unroll
       for (int ct = 0; ct < 2; ++ct)
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           const int j = 16 * ct + 4 * i + lq;
-          cx<T>* at = whole ? d.scratch + sm.piv[j] * n + to : J + j * ld + row;
-          if (j < w) gst(at, cx<T>{cre[rt][ct][i], cim[rt][ct][i]});
+          if (j < w) gst(J + j * ld + row, cx<T>{cre[rt][ct][i], cim[rt][ct][i]});
         }
     }
   }
-  if (live && h == 0 && !whole) roles[r] = role;
+  if (live && h == 0) roles[r] = role;
   if (tid < w) d.ipiv[p0 + tid] = sm.piv[tid];
   // info: reset by the first panel, then the first singular column wins
   if (sing != INT_MAX) atomicMin(&sm.sing, sing);
@@ -712,7 +709,6 @@ __global__ __launch_bounds__(4 * NMAX) void gj_panel_rows_kernel(const InvDesc<T
   __shared__ GjLds<T, WP> sm;
   const InvDesc<T> d = descs[blockIdx.x];
   const int n = d.n;
-  if (p0 >= n) return;                    // uniform: this block is already done
   const int64_t ld = d.ld;
   cx<T>* __restrict__ M = d.M;
   cx<T>* __restrict__ R = d.scratch;
@@ -741,7 +737,7 @@ __global__ __launch_bounds__(4 * NMAX) void gj_panel_rows_kernel(const InvDesc<T
   __syncthreads();                        // all pivot rows are in sm.piv
   // C -> M[:, J]; a block of one panel goes to its place in its final order,
   // A^{-1}[k, l] = C[r_k, r^{-1}(l)]
-  const bool whole = n <= WP;
+  const bool whole = NMAX <= 64 && n <= WP;
   if (live) {
 #pragma unroll
     for (int k = 0; k < CPT; ++k) {
@@ -782,23 +778,21 @@ __global__ __launch_bounds__(4 * NMAX) void gj_panel_rows_kernel(const InvDesc<T
 // M3 = false up to GJ_ROWS_MAX rows: the 3M product's error (relative to the product of
 // the norms and not entry by entry) shows there, residual of complex64 inverses over that of four
 // products 1.04 at 48 and 64 rows, 1.09 at 74 and 95, 1.12 at 112.
-template <class T, int S, bool M3>
+template <class T, bool M3>
 __global__ __launch_bounds__(256, 3) void gj_update_kernel(const InvDesc<T>* __restrict__ descs, int ndesc, int per,
                                                            int p0) {
-  constexpr int TS = 32 * S;
-  __shared__ GemmLds<T, S> sm;
+  constexpr int TS = 32;
+  __shared__ GemmLds<T, 1> sm;
   int di, t;
   xcd_item(blockIdx.x, per, ndesc, di, t);
   if (di >= ndesc) return;
   const InvDesc<T> v = descs[di];
   const int n = v.n;
-  if (p0 >= n) return;
   int q0, wo;
   gj_outer_range(n, p0, q0, wo);
   const int w = min(GJM_WP, n - p0);
   const int n0 = p0 - q0, n1 = q0 + wo - (p0 + w);
-  const int tm = (n + TS - 1) / TS, tn0 = (n0 + TS - 1) / TS, tn1 = (n1 + TS - 1) / TS;
-  if (t >= tm * (tn0 + tn1)) return;      // uniform over the workgroup
+  const int tm = (n + TS - 1) / TS, tn0 = n0 / TS;
   int jstart = q0, ncols = n0;
   if (t >= tm * tn0) {
     t -= tm * tn0;
@@ -820,7 +814,7 @@ __global__ __launch_bounds__(256, 3) void gj_update_kernel(const InvDesc<T>* __r
   d.n = ncols;
   d.alpha = T(1);
   d.beta = T(1);
-  gemm_tile_body<T, S, M3>(d, t, sm, reinterpret_cast<const int*>(v.scratch + (size_t)GJM_WP * n), p0);
+  gemm_tile_body<T, 1, M3>(d, t, sm, reinterpret_cast<const int*>(v.scratch + (size_t)GJM_WP * n), p0);
 }
 
 // S[l n + k] = M[r_k, r^{-1}(l)], the inverse in its final order and place.  Grid:
@@ -835,7 +829,6 @@ __global__ __launch_bounds__(256) void gj_perm_kernel(const InvDesc<T>* __restri
   __shared__ cx<T> sCol[4][512];
   const InvDesc<T> d = descs[blockIdx.y];
   const int n = d.n, l0 = blockIdx.x * cc;
-  if (l0 >= n || n <= GJM_WP) return;                      // blocks of one panel are in order already
   for (int j = threadIdx.x; j < n; j += 256) {
     const int rj = d.ipiv[j];
     sRow[j] = rj;
@@ -867,7 +860,6 @@ template <class T>
 __global__ __launch_bounds__(256) void gj_outer_gather_kernel(const InvDesc<T>* __restrict__ descs, int q0) {
   const InvDesc<T> d = descs[blockIdx.y];
   const int n = d.n;
-  if (n < GJ_OUTER_MIN || q0 >= n) return;
   const int wo = min(GJ_WO, n - q0);
   const int64_t ld = d.ld;
   cx<T>* __restrict__ M = d.M;
@@ -895,11 +887,9 @@ __global__ __launch_bounds__(256, 3) void gj_outer_update_kernel(const InvDesc<T
   if (di >= ndesc) return;
   const InvDesc<T> v = descs[di];
   const int n = v.n;
-  if (n < GJ_OUTER_MIN || q0 >= n) return;
   const int wo = min(GJ_WO, n - q0);
   const int n1 = n - q0 - wo;
-  const int tm = (n + TS - 1) / TS, tn0 = (q0 + TS - 1) / TS, tn1 = (n1 + TS - 1) / TS;
-  if (t >= tm * (tn0 + tn1)) return;      // uniform over the workgroup
+  const int tm = (n + TS - 1) / TS, tn0 = q0 / TS;
   int jstart = 0, ncols = q0;
   if (t >= tm * tn0) {
     t -= tm * tn0;
@@ -924,73 +914,76 @@ __global__ __launch_bounds__(256, 3) void gj_outer_update_kernel(const InvDesc<T
   gemm_tile_body<T, S>(d, t, sm, reinterpret_cast<const int*>(v.scratch + (size_t)GJM_WP * n), q0);
 }
 
-template <class T, int S>
-static void launch_gj_updates(const InvDesc<T>* d_descs, int ndesc, int nmax, int p0, hipStream_t s) {
-  constexpr int TS = 32 * S;
-  const int nt = (nmax + TS - 1) / TS;
-  // column tiles of the two ranges an update covers: at most 128 / TS + 1 in
-  // an outer panel of 128 columns, at most nt + 1 in a block below
-  // GJ_OUTER_MIN rows (whichever is more when a launch holds both)
-  const int ntb = ((nmax < GJ_OUTER_MIN ? nmax : GJ_OUTER_MIN) + TS - 1) / TS + 1;
-  const int per = nt * (nmax >= GJ_OUTER_MIN && ntb < GJ_WO / TS + 1 ? GJ_WO / TS + 1 : ntb);
-  if (sizeof(T) == 4 && nmax <= GJ_ROWS_MAX)
-    hipLaunchKernelGGL((gj_update_kernel<T, S, false>), dim3(xcd_grid(ndesc, per)), dim3(256), 0, s, d_descs, ndesc,
-                       per, p0);
-  else
-    hipLaunchKernelGGL((gj_update_kernel<T, S, true>), dim3(xcd_grid(ndesc, per)), dim3(256), 0, s, d_descs, ndesc,
-                       per, p0);
+// One workgroup per tile of the columns [q0, p0) and [p0 + w, q0 + wo) of an outer panel:
+// p0 - q0 is a multiple of the tile's 32, so that is one column of tiles less than the outer
+// panel has.
+template <class T>
+static void launch_gj_updates(const InvDesc<T>* d_descs, int ndesc, int n, int p0, hipStream_t s) {
+  const int q0 = n >= GJ_OUTER_MIN ? p0 / GJ_WO * GJ_WO : 0;
+  const int wo = n >= GJ_OUTER_MIN && n - q0 > GJ_WO ? GJ_WO : n - q0;
+  const int per = ((n + 31) / 32) * ((wo + 31) / 32 - 1);
+  if (per == 0) return;
+  const dim3 grid(xcd_grid(ndesc, per));
+  if constexpr (sizeof(T) == 4) {
+    if (n <= GJ_ROWS_MAX) {
+      hipLaunchKernelGGL((gj_update_kernel<T, false>), grid, dim3(256), 0, s, d_descs, ndesc, per, p0);
+      return;
+    }
+  }
+  hipLaunchKernelGGL((gj_update_kernel<T, true>), grid, dim3(256), 0, s, d_descs, ndesc, per, p0);
 }
 
+// The same for the columns [0, q0) and [q0 + wo, n); q0 is a multiple of 128.
 template <class T, int S>
-static void launch_gj_outer_updates(const InvDesc<T>* d_descs, int ndesc, int nmax, int q0, hipStream_t s) {
-  const int nt = (nmax + 32 * S - 1) / (32 * S), per = nt * nt;
+static void launch_gj_outer_updates(const InvDesc<T>* d_descs, int ndesc, int n, int q0, hipStream_t s) {
+  constexpr int TS = 32 * S;
+  const int n1 = n - q0 > GJ_WO ? n - q0 - GJ_WO : 0;
+  const int per = ((n + TS - 1) / TS) * (q0 / TS + (n1 + TS - 1) / TS);
   hipLaunchKernelGGL((gj_outer_update_kernel<T, S>), dim3(xcd_grid(ndesc, per)), dim3(256), 0, s, d_descs, ndesc, per,
                      q0);
 }
 
 template <class T>
-static hipError_t gj_inverse_launches(const InvDesc<T>* d_descs, int ndesc, int nmax, hipStream_t s) {
-  const int nt = (nmax + 63) / 64;
-  for (int p0 = 0; p0 < nmax; p0 += GJM_WP) {
+static hipError_t gj_inverse_launches(const InvDesc<T>* d_descs, int ndesc, int n, hipStream_t s) {
+  const int nt = (n + 63) / 64;
+  for (int p0 = 0; p0 < n; p0 += GJM_WP) {
     // the smallest workgroup that has the rows: fewer waves meet at a step's barriers
     // (an inversion of one block: complex64 300 rows, 384 instead of 512, 424 -> 388 us,
     // 374 rows 520 -> 477; complex128 150 rows, 192 instead of 256, 194 -> 189)
-    if (nmax <= 64)
-      hipLaunchKernelGGL((gj_panel_rows_kernel<T, 64>), dim3(ndesc), dim3(4 * 64), 0, s, d_descs, p0);
-    else if (nmax <= 96)
-      hipLaunchKernelGGL((gj_panel_rows_kernel<T, 96>), dim3(ndesc), dim3(4 * 96), 0, s, d_descs, p0);
-    else if (nmax <= GJ_ROWS_MAX)
-      hipLaunchKernelGGL((gj_panel_rows_kernel<T, GJ_ROWS_MAX>), dim3(ndesc), dim3(4 * GJ_ROWS_MAX), 0, s, d_descs, p0);
-    else if (nmax <= 128)
-      hipLaunchKernelGGL((gj_panel_kernel<T, 128>), dim3(ndesc), dim3(128 * GJ_TPR<T, 128>), 0, s, d_descs, p0);
-    else if (nmax <= 192)
-      hipLaunchKernelGGL((gj_panel_kernel<T, 192>), dim3(ndesc), dim3(192 * GJ_TPR<T, 192>), 0, s, d_descs, p0);
-    else if (nmax <= 256)
-      hipLaunchKernelGGL((gj_panel_kernel<T, 256>), dim3(ndesc), dim3(256 * GJ_TPR<T, 256>), 0, s, d_descs, p0);
-    else if (sizeof(T) == 4 && nmax <= 384)
-      hipLaunchKernelGGL((gj_panel_kernel<float, 384>), dim3(ndesc), dim3(384 * GJ_TPR<float, 384>), 0, s,
-                         reinterpret_cast<const InvDesc<float>*>(d_descs), p0);
-    else
-      hipLaunchKernelGGL((gj_panel_kernel<T, 512>), dim3(ndesc), dim3(512 * GJ_TPR<T, 512>), 0, s, d_descs, p0);
-    if (nmax <= GJM_WP) return hipGetLastError();          // one panel, stored in its final order
-    // the columns an update covers come in multiples of 32 (a panel's width)
-    launch_gj_updates<T, 1>(d_descs, ndesc, nmax, p0, s);
-    // the end of an outer panel (of every block whose outer panel holds p0)
+    auto rows = [&](auto nm) {
+      constexpr int NMAX = decltype(nm)::value;
+      hipLaunchKernelGGL((gj_panel_rows_kernel<T, NMAX>), dim3(ndesc), dim3(4 * NMAX), 0, s, d_descs, p0);
+    };
+    auto panel = [&](auto nm) {
+      constexpr int NMAX = decltype(nm)::value;
+      hipLaunchKernelGGL((gj_panel_kernel<T, NMAX>), dim3(ndesc), dim3(NMAX * GJ_TPR<T, NMAX>), 0, s, d_descs, p0);
+    };
+    constexpr int MID = sizeof(T) == 4 ? 384 : 512;
+    if (n <= 64) rows(std::integral_constant<int, 64>{});
+    else if (n <= 96) rows(std::integral_constant<int, 96>{});
+    else if (n <= GJ_ROWS_MAX) rows(std::integral_constant<int, GJ_ROWS_MAX>{});
+    else if (n <= 128) panel(std::integral_constant<int, 128>{});
+    else if (n <= 192) panel(std::integral_constant<int, 192>{});
+    else if (n <= 256) panel(std::integral_constant<int, 256>{});
+    else if (n <= MID) panel(std::integral_constant<int, MID>{});
+    else panel(std::integral_constant<int, 512>{});
+    if (n <= GJM_WP) return hipGetLastError();             // one panel, stored in its final order
+    launch_gj_updates<T>(d_descs, ndesc, n, p0, s);
     const int pe = p0 + GJM_WP;
-    if (nmax >= GJ_OUTER_MIN && (pe % GJ_WO == 0 || pe >= nmax)) {
+    if (n >= GJ_OUTER_MIN && (pe % GJ_WO == 0 || pe >= n)) {         // the end of an outer panel
       const int q0 = (p0 / GJ_WO) * GJ_WO;
-      const int chunks = (nmax * GJ_WO + 255) / 256 < 256 ? (nmax * GJ_WO + 255) / 256 : 256;
+      const int chunks = (n * GJ_WO + 255) / 256 < 256 ? (n * GJ_WO + 255) / 256 : 256;
       hipLaunchKernelGGL((gj_outer_gather_kernel<T>), dim3(chunks, ndesc), dim3(256), 0, s, d_descs, q0);
       if (gemm_small_tiles<T>(ndesc, nt * nt, 4 * nt * nt))
-        launch_gj_outer_updates<T, 1>(d_descs, ndesc, nmax, q0, s);
+        launch_gj_outer_updates<T, 1>(d_descs, ndesc, n, q0, s);
       else
-        launch_gj_outer_updates<T, 2>(d_descs, ndesc, nmax, q0, s);
+        launch_gj_outer_updates<T, 2>(d_descs, ndesc, n, q0, s);
     }
   }
   // four columns a workgroup (one a wave) on few blocks, 16 where that many
   // workgroups would mostly read the pivots
   const int cc = ndesc <= 32 ? 4 : 16;
-  hipLaunchKernelGGL((gj_perm_kernel<T>), dim3((nmax + cc - 1) / cc, ndesc), dim3(256), 0, s, d_descs, cc);
+  hipLaunchKernelGGL((gj_perm_kernel<T>), dim3((n + cc - 1) / cc, ndesc), dim3(256), 0, s, d_descs, cc);
   return hipGetLastError();
 }
 
@@ -1010,10 +1003,10 @@ hipError_t launch_gemm_batched(const GemmDesc<T>* d_descs, int ndesc, GemmTiles 
 }
 
 template <class T>
-hipError_t launch_gj_inverse(const InvDesc<T>* d_descs, int ndesc, int nmax, hipStream_t s) {
+hipError_t launch_gj_inverse(const InvDesc<T>* d_descs, int ndesc, int n, hipStream_t s) {
   if (ndesc <= 0) return hipSuccess;
-  if (nmax > 512) return hipErrorInvalidValue;
-  return gj_inverse_launches<T>(d_descs, ndesc, nmax, s);
+  if (n < 1 || n > 512) return hipErrorInvalidValue;
+  return gj_inverse_launches<T>(d_descs, ndesc, n, s);
 }
 
 template hipError_t launch_gemm_batched<double>(const GemmDesc<double>*, int, GemmTiles, hipStream_t);

@@ -746,8 +746,9 @@ hipError_t launch_skinny(const SkinnyDesc<T>* d_descs, int ndesc, int max_m, int
   // one or two columns from 400 workgroups of skinny_row_kernel (complex64: 37
   // blocks of 374 rows, 444 workgroups, 27 -> 23 us, 37 of 200 rows, 259, 9 -> 11;
   // complex128 with two columns 42 -> 40 at 888, with one 39 either way, so that
-  // stays).  Its lanes want two rows and more: a degree's block holds the rows of
-  // one to four fields, so a list whose largest block has 64 has none below 16.
+  // stays).  Its complex64 lanes read two rows, so no block may have just one: blocks
+  // differ by a factor of four at most (checked where the layout is built), so a list
+  // whose largest has 64 rows has none below 16.
   const dim3 wgrid((unsigned)((max_m + SKR_ROWS<T> - 1) / SKR_ROWS<T>), (unsigned)ndesc);
   const bool wide = max_m >= 64 && (int64_t)wgrid.x * wgrid.y >= 400;
   // blocks of 257 to 512 rows in at most one workgroup per CU: one memory round trip

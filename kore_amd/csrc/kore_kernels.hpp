@@ -50,9 +50,9 @@ struct GemmTiles {
 };
 template <class T>
 hipError_t launch_gemm_batched(const GemmDesc<T>* d_descs, int ndesc, GemmTiles t, hipStream_t s);
-// nmax: largest block size in the list (at most 512)
+// n: rows of every block of the list (at most 512)
 template <class T>
-hipError_t launch_gj_inverse(const InvDesc<T>* d_descs, int ndesc, int nmax, hipStream_t s);
+hipError_t launch_gj_inverse(const InvDesc<T>* d_descs, int ndesc, int n, hipStream_t s);
 template <class T>
 hipError_t launch_skinny(const SkinnyDesc<T>* d_descs, int ndesc, int max_m, int nrhs, hipStream_t s);
 // the same for one right-hand side, descriptors of at most np (= 1)

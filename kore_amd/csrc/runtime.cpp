@@ -551,6 +551,15 @@ static int32_t layout_build(const kore_layout* L, int64_t* sizmat, std::vector<i
     if (sz && sizes) sizes->push_back(sz);
   }
   if (perm && (int64_t)perm->size() != off) return fail(KORE_ERR_ARG, "internal: permutation size mismatch");
+  // what the factor's launches rest on: the blocks of a level's list, all of one
+  // parity, have one size (launch_gj_inverse), and no block has more than four times another's rows
+  // (launch_skinny, whose tail list holds both)
+  if (sizes && !sizes->empty()) {
+    const int s0 = (*sizes)[0], s1 = (*sizes)[sizes->size() > 1 ? 1 : 0];
+    for (size_t k = 0; k < sizes->size(); ++k)
+      if ((*sizes)[k] != (k & 1 ? s1 : s0) || s0 > 4 * s1 || s1 > 4 * s0)
+        return fail(KORE_ERR_ARG, "internal: degree blocks of sizes %d, %d and %d", s0, s1, (*sizes)[k]);
+  }
   return KORE_OK;
 }
 
@@ -571,7 +580,7 @@ struct FactorBase {
 
 template <class T> struct Level {
   InvDesc<T>* inv = nullptr;
-  int ninv = 0, maxn_inv = 0;
+  int ninv = 0, n_inv = 0;             // blocks, rows of each
   GemmDesc<T>* g1 = nullptr;
   int ng1 = 0;
   GemmTiles t1;
@@ -958,7 +967,7 @@ template <class T> static int32_t factor_build(kore_sys* s, Factor<T>* F) {
       vinv.push_back(InvDesc<T>{F->G[k], nk(k), (int)nk(k), ipiv + (size_t)k * nmax, F->info + k, F->D[k]});
       flops += 8.0 * nk(k) * nk(k) * nk(k);
       F->flops_inv += 8.0 * nk(k) * nk(k) * nk(k);
-      L.maxn_inv = std::max(L.maxn_inv, (int)nk(k));
+      L.n_inv = (int)nk(k);
     }
     rinv[l].n = vinv.size() - rinv[l].off;
     if (l == 0 && sp0) {
@@ -1335,7 +1344,7 @@ template <class T> static int32_t factor_run(kore_sys* s, Factor<T>* F) {
     Level<T>& L = F->lev[l];
     {
       Timed tm(c, KORE_TIMER_INV);
-      HIP_TRY(launch_gj_inverse<T>(L.inv, L.ninv, L.maxn_inv, st));
+      HIP_TRY(launch_gj_inverse<T>(L.inv, L.ninv, L.n_inv, st));
     }
     if (l == 0 && F->lev0_sparse) {
       Timed tm(c, KORE_TIMER_SPARSE);

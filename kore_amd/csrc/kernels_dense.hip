@@ -277,10 +277,11 @@ template <class T> __device__ __forceinline__ T tiny_pivot() { return sizeof(T) 
 //   gj_update_kernel  M[i, j] <- [i not in P] M[i, j] + sum_k C[i, k] R[k, j]
 //                     for j outside J, on matrix cores;
 // then gj_perm_kernel: A^{-1}[k, l] = M[r_k, r^{-1}(l)] into the scratch block,
-// which is where the inverse is wanted.  Blocks of one panel (up to 32 rows) are complete
-// after gj_panel_kernel, which stores them in their final order: one launch
+// which is where the inverse is wanted.  Blocks of up to 112 rows take
+// gj_panel_rows_kernel for the panel; those of one panel (up to 32 rows) are complete
+// after it, which stores them in their final order: one launch
 // (24 rows, complex128: 55 -> 19 us; a kernel that ran the whole elimination of
-// a block in one workgroup, used below 96 rows, is gone: 74 rows 193 -> 82 us).
+// a block in one workgroup, used below 96 rows, is gone: 74 rows 193 -> 86 us).
 // Scratch layout (per block of more than 32 rows, n x n complex): R
 // (32 x n, R[k, j] at R[j 32 + k]), then n ints of row roles (-1 unused,
 // c >= 0: the pivot row of column c).  The multi-panel composition: with T
@@ -700,8 +701,8 @@ __global__ __launch_bounds__((NMAX * GJ_TPR<T, NMAX>), (sizeof(T) == 4 ? 4 : 2))
 // at 97 rows over the earlier panel kernel, which updated all 32 columns by fused
 // multiply-adds; from 104 rows on 0.99.  This form: 0.99 to 1.00, and 0.95 at 96 to 112 rows.
 // Up to 64 rows it is the faster one too (64 rows 59 against 63 us, complex64 51 against 57);
-// above it costs a tenth: 74 rows 84 -> 90 us, 95 rows 100 -> 112, 112 rows 120 -> 142 in
-// complex128, 74 -> 78, 87 -> 94 and 106 -> 118 in complex64.
+// above it costs up to a seventh: 74 rows 84 -> 90 us, 95 rows 100 -> 112, 112 rows 119 -> 138 in
+// complex128, 74 -> 78, 86 -> 93 and 106 -> 118 in complex64.
 constexpr int GJ_ROWS_MAX = 112;
 template <class T, int NMAX>
 __global__ __launch_bounds__(4 * NMAX) void gj_panel_rows_kernel(const InvDesc<T>* __restrict__ descs, int p0) {

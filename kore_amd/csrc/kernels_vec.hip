@@ -765,9 +765,15 @@ hipError_t launch_skinny(const SkinnyDesc<T>* d_descs, int ndesc, int max_m, int
   // the preloading form at every size: measured no slower than the streaming
   // loop on the largest sweep levels (thousands of workgroups) and faster on
   // the deep levels, where a launch holds a handful of blocks.  Three or four
-  // columns of blocks of 129 to 256 rows stay on it too (complex64, 200 rows, 150
-  // blocks of two products: 31 us against 36 on the matrix cores; 100 rows 16
-  // against 15, 374 rows, 37 blocks 45 against 31)
+  // columns of blocks of 129 to 256 rows stay on it too.  Two products, four columns, us
+  // per launch on it / on the matrix cores: complex128 160 rows one block 7.7 / 8.1, 37
+  // blocks 11.0 / 14.6, 150 blocks 33 / 40; 200 rows 7.8 / 7.9, 14.1 / 15.7, 44 / 50; complex64
+  // 160 rows 6.5 / 6.3, 8.1 / 10.0, 19.5 / 24.7; 200 rows 6.6 / 6.2, 10.3 / 11.1, 29 /
+  // 32; at 256 rows the matrix cores take 0 to 1.3 us less (complex128 150 blocks 71 / 65).  Outside
+  // that range they are faster nearly everywhere: complex128 64 rows 7.4 / 5.6, 7.8 / 5.9,
+  // 14 / 12; 128 rows 7.6 / 5.0, 9.1 / 7.5, 28 / 21; 257 rows 10.1 / 8.5, 32 / 29, 94 / 86;
+  // complex64 128 rows 6.4 / 4.1, 7.4 / 5.9, 16 / 12, 300 rows 9.4 / 7.8, 21.4 / 21.1, 73 / 64
+  // (slower: complex128 300 rows 19 blocks 19.3 / 20.7, complex64 64 rows 150 blocks 7.8 / 8.5).
   if constexpr (sizeof(T) == 4) {
     if (wide && nrhs == 1) {
       hipLaunchKernelGGL((skinny_row_kernel<T, 1>), wgrid, dim3(64 * SKR_NW), 0, s, d_descs, nrhs);
